@@ -2,8 +2,9 @@
 // the top-k combine, and the whole vLLM MoE layer (vllm:233-265).
 //
 // Routing (the format of vllm:119-146, consumed as soft:101-108) is built
-// without any host synchronisation in three deterministic passes over
-// 1024-route chunks:
+// without any host synchronisation, up to 16384 routes in one launch
+// (align_one), beyond that in three deterministic passes over 1024-route
+// chunks (the last two one launch up to 64 chunks):
 //   count  -- per-chunk expert histogram (LDS atomics; counts only);
 //   scan   -- one workgroup turns the histograms into, for every (chunk,
 //             expert), the absolute position of that chunk's first route of
@@ -25,21 +26,11 @@ namespace mx {
 namespace {
 
 constexpr int kChunk = 1024;  // routes per count/place workgroup
-// Routes the single-workgroup routing handles: up to kSingle one 256-thread
-// workgroup; up to kSingleWide one 1024-thread workgroup (4096 routes: ~6
-// us in the kernel against 15.4 us of kernel time for the three launches;
-// for up to 1024 routes, 256 threads beat 1024: 5.0 vs 5.4 us).
-constexpr int kSingle = 1024;
-constexpr int kSingleWide = 4096;
 // Layers with at most this many routes use direct routing in the GEMMs
 // (no kernel builds sorted metadata); must not exceed the skinny kernel's
 // scan limit (256).
 constexpr int64_t kDirectRoutes = 64;
 constexpr int kMaxExperts = 1024;
-// Experts the single-workgroup routing kernel holds in LDS (more use the
-// three-launch path).
-constexpr int kSingleExperts = 256;
-
 // Expert of a route: its id when in [0, num_experts), else drop_to.  With
 // drop_to = -1 the route is dropped (in no block; its output rows are not
 // written).  The fused soft op passes num_experts = E + 1 and drop_to = E:
@@ -198,6 +189,134 @@ __global__ __launch_bounds__(256) void align_place(const TI* __restrict__ ids, i
   }
 }
 
+// The whole routing in one launch, for at most kOneLaunch routes: workgroup c
+// places the kOneChunk routes of chunk c and derives what it needs from the
+// ids themselves -- every workgroup counts all routes before and after its
+// chunk per expert (coalesced loads, LDS atomics) -- so no workgroup waits
+// for another and no counts pass through memory.  Then the padded exclusive
+// scan over the experts; the lanes of a wave with the same expert come from
+// ballots (one per id bit), their counts become each wave's first position
+// per expert, and every route lands at its wave's position + its rank among
+// the lower lanes: route order within an expert.  Workgroup c also writes,
+// by whole waves, expert_ids and the sentinel padding of the experts x with
+// x % gridDim.x == c, and workgroup 0 the padded route count; small routings
+// launch kOneLeast workgroups for that (with one, its 8 waves walk 16
+// experts' padding each: 256 routes 7.9 us, with 16 to 64 workgroups 4.3).
+// Latency bound: one round of id loads, three barriers, one round of
+// stores.  Graph replays of the call, 128 experts, 64-row blocks, 256 / 1024
+// / 4096 / 8000 / 16384 routes: 4.3 / 4.5 / 4.9 / 5.5 / 7.3 us, against 5.7 /
+// 6.2 / 6.5 us in one workgroup (all phases on one CU) and 7.9 / 7.8 us for
+// the count and scan + place launches, which win above (32768 routes: 10.4
+// us here, where every workgroup counts every id, against 7.8).
+constexpr int kOneChunk = 512;
+constexpr int64_t kOneLeast = 16;
+constexpr int64_t kOneLaunch = 16384;
+
+template <typename TI>
+__global__ __launch_bounds__(kOneChunk) void align_one(const TI* __restrict__ ids, int64_t n,
+                                                       int num_experts, int drop_to, int id_bits,
+                                                       int block_m,
+                                                       int32_t* __restrict__ sorted_ids,
+                                                       int32_t* __restrict__ expert_ids,
+                                                       int32_t* __restrict__ num_post_padded) {
+  constexpr int NT = kOneChunk, W = NT / 64;
+  constexpr int EPT = kMaxExperts / NT;  // experts per thread in the scan
+  constexpr int B = 16;                  // id loads per thread per round trip
+  __shared__ int wpos[W * kMaxExperts];  // [wave][expert]: counts, then next positions
+  // routes of earlier / later chunks; then first slot / first sentinel slot
+  __shared__ int s_pre[kMaxExperts], s_post[kMaxExperts];
+  __shared__ int part[W];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  const int c = (int)blockIdx.x, nwg = (int)gridDim.x;
+  const int ne = num_experts;
+  const int64_t mine = (int64_t)c * NT + tid;
+  const int eid = mine < n ? route_expert(ids[mine], ne, drop_to) : -1;
+  TI v[B];
+#pragma unroll
+  for (int b = 0; b < B; ++b) v[b] = (int64_t)b * NT + tid < n ? ids[b * NT + tid] : (TI)0;
+  for (int i = tid; i < W * ne; i += NT) wpos[i] = 0;
+  for (int x = tid; x < ne; x += NT) s_pre[x] = s_post[x] = 0;
+  __syncthreads();
+  for (int64_t i0 = 0; i0 < n; i0 += B * NT) {
+    if (i0 > 0) {
+#pragma unroll
+      for (int b = 0; b < B; ++b) {
+        const int64_t r = i0 + b * NT + tid;
+        v[b] = r < n ? ids[r] : (TI)0;
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      const int cc = (int)(i0 / NT) + b;
+      if (cc == c || i0 + b * NT + tid >= n) continue;
+      const int e = route_expert(v[b], ne, drop_to);
+      if (e >= 0) atomicAdd(cc < c ? &s_pre[e] : &s_post[e], 1);
+    }
+  }
+  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  uint64_t same = __ballot(eid >= 0);
+  for (int bit = 0; bit < id_bits; ++bit) {
+    const bool b = (eid >> bit) & 1;  // lanes of invalid ids are out of every mask
+    const uint64_t bal = __ballot(b);
+    same &= b ? bal : ~bal;
+  }
+  const int rank = __popcll(same & lt_mask);
+  if (eid >= 0 && rank == 0) wpos[wave * ne + eid] = __popcll(same);
+  __syncthreads();
+  // padded exclusive scan over the experts (thread-local EPT, wave shuffles,
+  // then the wave sums)
+  int tot[EPT], pad[EPT], local = 0;
+#pragma unroll
+  for (int jj = 0; jj < EPT; ++jj) {
+    const int x = tid * EPT + jj;
+    tot[jj] = 0;
+    if (x < ne) {
+      tot[jj] = s_pre[x] + s_post[x];
+#pragma unroll
+      for (int w = 0; w < W; ++w) tot[jj] += wpos[w * ne + x];
+    }
+    pad[jj] = (tot[jj] + block_m - 1) / block_m * block_m;
+    local += pad[jj];
+  }
+  int sum = local;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int u = __shfl_up(sum, off);
+    if (lane >= off) sum += u;
+  }
+  if (lane == 63) part[wave] = sum;
+  __syncthreads();
+  for (int w = 0; w < wave; ++w) sum += part[w];
+  int start = sum - local;
+#pragma unroll
+  for (int jj = 0; jj < EPT; ++jj) {
+    const int x = tid * EPT + jj;
+    if (x < ne) {
+      int p = start + s_pre[x];
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        const int cw = wpos[w * ne + x];
+        wpos[w * ne + x] = p;
+        p += cw;
+      }
+      s_pre[x] = start;
+      s_post[x] = start + tot[jj];
+    }
+    start += pad[jj];
+  }
+  if (c == 0 && tid == NT - 1) num_post_padded[0] = sum;
+  __syncthreads();
+  if (eid >= 0) sorted_ids[wpos[wave * ne + eid] + rank] = (int32_t)mine;
+  for (int x = c + wave * nwg; x < ne; x += W * nwg) {
+    const int st = s_pre[x], fill = s_post[x];
+    const int blocks = (fill - st + block_m - 1) / block_m;
+    for (int i = lane; i < blocks; i += 64) expert_ids[st / block_m + i] = x;
+    for (int q = fill + lane; q < st + blocks * block_m; q += 64) sorted_ids[q] = (int32_t)n;
+  }
+}
+
 // Scan and placement in one launch, after align_count, for at most
 // kScanPlaceChunks chunks: workgroup c places chunk c's kChunk routes and
 // first derives what it needs from the per-chunk counts itself -- for each
@@ -205,7 +324,7 @@ __global__ __launch_bounds__(256) void align_place(const TI* __restrict__ ids, i
 // loads, summed with LDS atomics), the padded exclusive scan over the
 // experts -- instead of waiting for a separate scan launch (redundant work
 // of nchunks x E count loads per workgroup, all L2 hits).  Placement as in
-// align_single: wave w owns routes w * RPT * 64 .. +RPT * 64 of the chunk,
+// align_one: wave w owns routes w * RPT * 64 .. +RPT * 64 of the chunk,
 // the lanes of a sub-chunk with the same expert come from ballots, per-wave
 // counts become per-wave positions, and each wave then places its
 // sub-chunks in order without barriers.  Workgroup c also writes, by whole
@@ -386,171 +505,6 @@ __global__ __launch_bounds__(256) void topk_sum(const T* __restrict__ d, const T
   }
 }
 
-// All three passes in one workgroup of NT threads for at most NT * RPT
-// routes and kSingleExperts experts (decode and small prefill).  Wave w owns
-// routes w * RPT * 64 .. +RPT * 64 in RPT sub-chunks of 64, so route order
-// is wave, then sub-chunk, then lane.  (1) Each lane finds the lanes of its
-// sub-chunk with the same expert (one ballot per id bit; the masks are kept
-// for step 3) and the lowest of them adds their count to the wave's row of
-// per-expert counts.  (2) One thread per expert sums its wave counts, the
-// padded sizes are scanned over the experts, and the wave rows become each
-// wave's first position per expert; expert ids and sentinel padding are
-// written.  (3) Every route lands at its wave's position for its expert +
-// its rank among the lower lanes, and the lowest lane advances the position
-// for the next sub-chunk -- route order within an expert, as align_place.
-// Three barriers in all (the placement needs none: a wave's LDS accesses
-// are ordered); 4096 routes: 9.1 -> 5.9 us, 1024: 7.7 -> 5.0 us of
-// in-kernel time against per-chunk placement over the whole workgroup.
-// When the padded routing fits kStageIds entries, the sentinel fill and the
-// placement write an LDS copy of sorted_ids, which then goes out in
-// coalesced stores instead of scattered ones (two more barriers; graph
-// replays of the call, 4096 routes over 129 experts: 7.16 -> 6.42 us, 1024
-// routes: 5.41 -> 4.94 us).
-constexpr int kStageIds = 12288;
-template <typename TI, int NT, int RPT>
-__global__ __launch_bounds__(NT) void align_single(const TI* __restrict__ ids, int64_t n,
-                                                   int num_experts, int drop_to, int id_bits,
-                                                   int block_m,
-                                                   int32_t* __restrict__ sorted_ids,
-                                                   int32_t* __restrict__ expert_ids,
-                                                   int32_t* __restrict__ num_post_padded) {
-  constexpr int W = NT / 64;                // waves
-  constexpr int E = kSingleExperts;
-  constexpr int EPT = (E + NT - 1) / NT;    // experts per thread in the scan
-  __shared__ int wpos[W][E];                // per-wave counts, then next positions
-  __shared__ int part[W];
-  __shared__ int s_fill[E], s_end[E];       // first sentinel slot, end of the padded range
-  __shared__ int s_total;
-  __shared__ int32_t s_ids[kStageIds];      // staged sorted_ids (padded total <= kStageIds)
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  int eid[RPT];
-  const int64_t rbase = (int64_t)wave * (RPT * 64);
-#pragma unroll
-  for (int j = 0; j < RPT; ++j) {
-    const int64_t r = rbase + j * 64 + lane;
-    eid[j] = r < n ? route_expert(ids[r], num_experts, drop_to) : -1;
-  }
-  for (int i = tid; i < W * E; i += NT) (&wpos[0][0])[i] = 0;
-  __syncthreads();
-  // (1) lanes of the sub-chunk with the same expert; the RPT ballot chains
-  // are independent, so they are interleaved bit by bit
-  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  uint64_t same[RPT];
-#pragma unroll
-  for (int j = 0; j < RPT; ++j) same[j] = __ballot(eid[j] >= 0);
-  for (int bit = 0; bit < id_bits; ++bit) {
-#pragma unroll
-    for (int j = 0; j < RPT; ++j) {
-      const bool b = (eid[j] >> bit) & 1;  // lanes of invalid ids are out of every mask
-      const uint64_t bal = __ballot(b);
-      same[j] &= b ? bal : ~bal;
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < RPT; ++j)
-    if (eid[j] >= 0 && __popcll(same[j] & lt_mask) == 0) wpos[wave][eid[j]] += __popcll(same[j]);
-  __syncthreads();
-  // (2) padded exclusive scan: thread tid owns experts tid*EPT .. +EPT; the
-  // per-thread totals are scanned with wave shuffles, then the wave sums
-  int cnt[EPT], pad[EPT], local = 0;
-#pragma unroll
-  for (int jj = 0; jj < EPT; ++jj) {
-    const int x = tid * EPT + jj;
-    int c = 0;
-    if (x < num_experts) {
-      int cw[W];  // all reads first: one LDS round trip, not W
-#pragma unroll
-      for (int w = 0; w < W; ++w) cw[w] = wpos[w][x];
-#pragma unroll
-      for (int w = 0; w < W; ++w) c += cw[w];
-    }
-    cnt[jj] = c;
-    pad[jj] = (c + block_m - 1) / block_m * block_m;
-    local += pad[jj];
-  }
-  int v = local;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int u = __shfl_up(v, off);
-    if (lane >= off) v += u;
-  }
-  if (lane == 63) part[wave] = v;
-  __syncthreads();
-  for (int w = 0; w < wave; ++w) v += part[w];
-  int start = v - local;
-#pragma unroll
-  for (int jj = 0; jj < EPT; ++jj) {
-    const int x = tid * EPT + jj;
-    if (x < num_experts) {
-      int p = start;
-#pragma unroll
-      for (int w = 0; w < W; ++w) {
-        const int c = wpos[w][x];
-        wpos[w][x] = p;
-        p += c;
-      }
-      for (int blk = start / block_m; blk < (start + pad[jj]) / block_m; ++blk) expert_ids[blk] = x;
-      s_fill[x] = start + cnt[jj];
-      s_end[x] = start + pad[jj];
-    }
-    start += pad[jj];
-  }
-  if (tid == NT - 1) {
-    num_post_padded[0] = v;
-    s_total = v;
-  }
-  __syncthreads();
-  const int total = s_total;
-  if (total <= kStageIds) {
-    for (int i = tid; i < total; i += NT) s_ids[i] = (int32_t)n;
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < RPT; ++j) {
-      if (rbase + j * 64 >= n) break;  // the same for the whole wave
-      if (eid[j] >= 0) {
-        const int e = eid[j];
-        const int rank = __popcll(same[j] & lt_mask);
-        const int base = wpos[wave][e];
-        s_ids[base + rank] = (int32_t)(rbase + j * 64 + lane);
-        if (rank == 0) wpos[wave][e] = base + __popcll(same[j]);
-      }
-    }
-    __syncthreads();
-    for (int i = tid; i < total; i += NT) sorted_ids[i] = s_ids[i];
-    return;
-  }
-  // sentinel padding (at most block_m - 1 slots per expert): consecutive
-  // lanes on consecutive slots of one expert
-  if ((block_m & (block_m - 1)) == 0) {
-    const int sh = __builtin_ctz(block_m);
-    for (int i = tid; i < num_experts * block_m; i += NT) {
-      const int x = i >> sh;
-      const int q = s_fill[x] + (i & (block_m - 1));
-      if (q < s_end[x]) sorted_ids[q] = (int32_t)n;
-    }
-  } else {
-    for (int i = tid; i < num_experts * block_m; i += NT) {
-      const int x = i / block_m;
-      const int q = s_fill[x] + (i - x * block_m);
-      if (q < s_end[x]) sorted_ids[q] = (int32_t)n;
-    }
-  }
-  // (3) placement
-#pragma unroll
-  for (int j = 0; j < RPT; ++j) {
-    if (rbase + j * 64 >= n) break;  // the same for the whole wave
-    if (eid[j] >= 0) {
-      const int e = eid[j];
-      const int rank = __popcll(same[j] & lt_mask);
-      const int base = wpos[wave][e];
-      sorted_ids[base + rank] = (int32_t)(rbase + j * 64 + lane);
-      if (rank == 0) wpos[wave][e] = base + __popcll(same[j]);
-    }
-  }
-}
-
 int64_t round_up(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
 
 void align_capacity(int64_t n, int num_experts, int block_m, int64_t* max_sorted,
@@ -582,14 +536,9 @@ int launch_align(const TI* ids, int64_t n, int num_experts, int drop_to, int blo
                  int64_t nchunks, hipStream_t st) {
   int id_bits = 0;
   while ((1 << id_bits) < num_experts) ++id_bits;
-  const bool single = num_experts <= kSingleExperts;
-  if (single && n <= kSingle) {
-    align_single<TI, 256, kSingle / 256><<<1, 256, 0, st>>>(
-        ids, n, num_experts, drop_to, id_bits, block_m, sorted_ids, expert_ids, npp);
-    return launch_status("align launch");
-  }
-  if (single && n <= kSingleWide) {
-    align_single<TI, 1024, kSingleWide / 1024><<<1, 1024, 0, st>>>(
+  if (n <= kOneLaunch) {
+    const int64_t chunks = (n + kOneChunk - 1) / kOneChunk;
+    align_one<TI><<<(unsigned)(chunks > kOneLeast ? chunks : kOneLeast), kOneChunk, 0, st>>>(
         ids, n, num_experts, drop_to, id_bits, block_m, sorted_ids, expert_ids, npp);
     return launch_status("align launch");
   }
