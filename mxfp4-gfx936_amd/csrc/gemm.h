@@ -75,6 +75,9 @@ struct GemmArgs {
   // block-scaled (W4A4) GEMMs: activation format, 0 = packed E2M1, 1 = FP8
   // E4M3, 2 = FP8 E5M2 (FP8 rows are k bytes)
   int32_t a_fp8;
+  // routed W4A16: run w4a16_dr (weights straight into registers); set where
+  // dr_supported and dr_faster hold
+  int32_t dr;
   // routed plain epilogues: scale as the reference's safe MoE path rounds
   // (ref_scaled) instead of once
   int32_t ref_round;
@@ -220,6 +223,10 @@ bool pf_prepacked_usable(const GemmArgs& g);
 int device_cus();
 int pf_choose(const GemmArgs& g, int epi);
 int launch_w4a16_pf(const GemmArgs& g, int dtype, int epi, int cfg, hipStream_t st);
+// Routed GEMM with the weights straight into registers (gemm_w4a16_dr.hip).
+bool dr_supported(const GemmArgs& g);
+bool dr_faster(int64_t routes, int64_t experts, int64_t n, int64_t k, bool silu, bool prepacked);
+int launch_w4a16_dr(const GemmArgs& g, int dtype, int epi, hipStream_t st);
 // Split-K plan for a dense plain-epilogue GEMM whose tiles would not fill
 // the chip: the tile configuration and slice count (1 = no split).
 struct SplitPlan {

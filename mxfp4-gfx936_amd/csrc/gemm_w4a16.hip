@@ -970,6 +970,7 @@ int launch_typed(const GemmArgs& g, hipStream_t st) {
     return launch_status("w4a16 skinny launch");
   }
   const int dt = std::is_same<T, __bf16>::value ? MXFP4_DT_BF16 : MXFP4_DT_F16;
+  if (g.dr) return launch_w4a16_dr(g, dt, EPI, st);
   if (pf_supported(g, (int)sizeof(T))) {
     // dense GEMMs too small to fill the chip split K when given a workspace
     if (EPI == EPI_STORE && !routed && g.splitk_ws != nullptr) {
@@ -1021,6 +1022,7 @@ int launch_w4a16(const GemmArgs& g, int dtype, int epi, hipStream_t st) {
       set_error("w4a16: C in FP32 needs bf16 activations on routed blocks of 32k rows");
       return MXFP4_ERR_VALUE;
     }
+    if (g.dr) return launch_w4a16_dr(g, dtype, epi, st);
     return launch_w4a16_pf(g, MXFP4_DT_BF16, EPI_STORE_F32, pf_choose(g, EPI_STORE), st);
   }
   if (dtype == MXFP4_DT_BF16)

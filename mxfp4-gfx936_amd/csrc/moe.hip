@@ -626,7 +626,7 @@ struct LayerPlan {
 };
 
 LayerPlan plan_layer(int64_t m, int top_k, int num_experts, int64_t hidden, int64_t inter,
-                     int64_t esize, bool prepacked) {
+                     int64_t esize, bool prepacked, bool dr) {
   LayerPlan p;
   p.routes = m * top_k;
   const double avg = (double)p.routes / (double)num_experts;
@@ -655,6 +655,7 @@ LayerPlan plan_layer(int64_t m, int top_k, int num_experts, int64_t hidden, int6
   // 88.4 / 94.8 vs 92.1 / 93.4 / 97.2 / 98.5 us with 32 rows; the
   // prepacked layer keeps 32 rows: 75.0-78.1 vs 82.2-94.8 us).
   if (!prepacked) p.block_m = avg <= 6.0 ? 16 : (avg <= 28.0 ? 32 : (avg <= 56.0 ? 64 : 128));
+  if (dr) p.block_m = 64;  // w4a16_dr
   align_capacity(p.routes, num_experts, p.block_m, &p.max_sorted, &p.max_blocks, &p.nchunks);
   int64_t off = 0;
   p.off_counts = off; off = round_up(off + (p.nchunks > 0 ? p.nchunks : 1) * num_experts * 4, 256);
@@ -863,9 +864,9 @@ struct SoftPlan {
   int64_t off_counts, off_sorted, off_experts, off_npp, total;
 };
 
-SoftPlan plan_soft(int64_t routes, int64_t num_experts, SoftPath path, int64_t k) {
+SoftPlan plan_soft(int64_t routes, int64_t num_experts, SoftPath path, int64_t k, bool dr) {
   SoftPlan p;
-  p.block_m = soft_block_m(routes, num_experts, path, k);
+  p.block_m = dr ? 64 : soft_block_m(routes, num_experts, path, k);
   p.zero_c = num_experts + 1 > kMaxExperts;
   p.align_experts = (int)(p.zero_c ? num_experts : num_experts + 1);
   p.drop_to = p.zero_c ? -1 : (int)num_experts;
@@ -941,6 +942,9 @@ extern "C" int mxfp4_moe_gemm_pre(const void* a, int a_dtype, int64_t a_rows,
                            c_row_stride, a_scale, b_scale, topk_weights, mul_routed_weight,
                            sorted_ids, expert_ids, num_post_padded, em, block_m, num_valid, top_k);
   set_prepacked(g, pre_b, pre_s, n, k);
+  const SoftPath path = soft_path(a_dtype, c_dtype, pre_b != nullptr);
+  g.dr = (path == SOFT_W4A16 || path == SOFT_F32_W4A16) && block_m % 32 == 0 && dr_supported(g) &&
+         dr_faster(num_valid, num_experts, n, k, false, false);
   return dispatch_gemm(g, a_dtype, c_dtype, EPI_STORE, static_cast<hipStream_t>(stream));
 }
 
@@ -953,13 +957,15 @@ extern "C" int mxfp4_fused_moe_workspace_size(int64_t m, int top_k, int64_t num_
     return MXFP4_ERR_VALUE;
   }
   // every plan fits: either layout (the caller may pass a prepacked copy),
-  // any K
+  // any K, w4a16_dr or not
   int64_t most = 0;
   for (int pre = 0; pre < 2; ++pre)
-    for (int64_t k : {(int64_t)0, (int64_t)1 << 30}) {
-      const int64_t t = plan_soft(m * top_k, num_experts, soft_path(a_dtype, c_dtype, pre), k).total;
-      most = t > most ? t : most;
-    }
+    for (int64_t k : {(int64_t)0, (int64_t)1 << 30})
+      for (int dr = 0; dr < 2; ++dr) {
+        const int64_t t =
+            plan_soft(m * top_k, num_experts, soft_path(a_dtype, c_dtype, pre), k, dr).total;
+        most = t > most ? t : most;
+      }
   *bytes = most;
   return MXFP4_OK;
 }
@@ -1000,14 +1006,26 @@ extern "C" int mxfp4_fused_moe_pre(const void* a, int a_dtype, int64_t a_rows,
     return MXFP4_ERR_VALUE;
   }
   const int64_t routes = m * top_k;
-  const SoftPlan p =
-      plan_soft(routes, num_experts, soft_path(a_dtype, c_dtype, pre_b != nullptr), k);
+  const SoftPath path = soft_path(a_dtype, c_dtype, pre_b != nullptr);
+  SoftPlan p = plan_soft(routes, num_experts, path, k, false);
   int rc = check_routed_args(a, a_dtype, a_row_stride, a_mx, b, num_experts, n, k, c_dtype, top_k,
                              p.block_m, p.max_sorted);
   if (rc) return rc;
   if (!aligned16(c)) {
     set_error("fused moe: C must be 16-byte aligned");
     return MXFP4_ERR_VALUE;
+  }
+  // checkpoint-layout weights on 64-row blocks of w4a16_dr where it is faster
+  // and its routing fits the workspace
+  bool dr = false;
+  if ((path == SOFT_W4A16 || path == SOFT_F32_W4A16) && routes > 0 && routes > kDirectRoutes) {
+    const GemmArgs g = routed_args(a, a_rows, a_row_stride, a_mx, b, b_mx, num_experts, n, k, c, n,
+                                   a_scale, b_scale, topk_weights, mul_routed_weight, nullptr,
+                                   nullptr, nullptr, routes, 64, routes, top_k);
+    const SoftPlan q = plan_soft(routes, num_experts, path, k, true);
+    dr = dr_supported(g) && dr_faster(routes, num_experts, n, k, false, false) &&
+         workspace_bytes >= q.total;
+    if (dr) p = q;
   }
   if (workspace_bytes < p.total || (p.total > 0 && !aligned16(workspace))) {
     set_error("fused moe: workspace too small or misaligned (%lld < %lld bytes)",
@@ -1019,7 +1037,6 @@ extern "C" int mxfp4_fused_moe_pre(const void* a, int a_dtype, int64_t a_rows,
   // Few routes on the W4A16 path: the decode kernels find each route's rows
   // from the top-k ids (direct routing, as in the MoE layer), so no routing
   // launch; a route whose id is outside [0, E) writes zeros to its row.
-  const SoftPath path = soft_path(a_dtype, c_dtype, pre_b != nullptr);
   const int64_t lim = (int64_t)1 << 31;
   if ((path == SOFT_W4A16 || path == SOFT_W4A16_PRE) && routes <= kDirectRoutes &&
       n * (k / 2) < lim && a_rows * a_row_stride * elem_size(a_dtype) < lim) {
@@ -1050,6 +1067,7 @@ extern "C" int mxfp4_fused_moe_pre(const void* a, int a_dtype, int64_t a_rows,
                            a_scale, b_scale, topk_weights, mul_routed_weight, sorted, experts, npp,
                            p.max_sorted, p.block_m, routes, top_k);
   set_prepacked(g, pre_b, pre_s, n, k);
+  g.dr = dr;
   return dispatch_gemm(g, a_dtype, c_dtype, EPI_STORE, st);
 }
 
@@ -1171,6 +1189,16 @@ extern "C" int mxfp4_linear_w4a4(const uint8_t* a, const uint8_t* a_mx, int64_t 
   return launch_w4a4(g, out_dtype, static_cast<hipStream_t>(stream));
 }
 
+namespace {
+// What the layer cannot do without: the larger of the two layouts' plans on
+// the prefill tiles' block sizes.
+int64_t layer_bytes(int64_t m, int top_k, int num_experts, int64_t hidden, int64_t inter) {
+  const int64_t a = plan_layer(m, top_k, num_experts, hidden, inter, 2, true, false).total;
+  const int64_t b = plan_layer(m, top_k, num_experts, hidden, inter, 2, false, false).total;
+  return a > b ? a : b;
+}
+}  // namespace
+
 extern "C" int mxfp4_moe_layer_workspace_size(int64_t m, int top_k, int num_experts,
                                               int64_t hidden, int64_t inter, int64_t* bytes) {
   if (m < 0 || top_k < 1 || num_experts < 1 || num_experts > kMaxExperts || hidden <= 0 ||
@@ -1178,10 +1206,11 @@ extern "C" int mxfp4_moe_layer_workspace_size(int64_t m, int top_k, int num_expe
     set_error("moe layer: invalid sizes");
     return MXFP4_ERR_VALUE;
   }
-  // either weight layout's plan fits (the caller may pass prepacked copies)
-  const int64_t a = plan_layer(m, top_k, num_experts, hidden, inter, 2, true).total;
-  const int64_t b = plan_layer(m, top_k, num_experts, hidden, inter, 2, false).total;
-  *bytes = a > b ? a : b;
+  // every plan fits: either weight layout (the caller may pass prepacked
+  // copies), w4a16_dr or not
+  const int64_t least = layer_bytes(m, top_k, num_experts, hidden, inter);
+  const int64_t dr = plan_layer(m, top_k, num_experts, hidden, inter, 2, true, true).total;
+  *bytes = least > dr ? least : dr;
   return MXFP4_OK;
 }
 
@@ -1223,7 +1252,7 @@ extern "C" int mxfp4_moe_layer_pre(const void* x, int x_dtype, int64_t m, int64_
     set_error("moe layer: buffers must be 16-byte aligned");
     return MXFP4_ERR_VALUE;
   }
-  const LayerPlan p = plan_layer(m, top_k, num_experts, hidden, inter, 2, pre13_b != nullptr);
+  LayerPlan p = plan_layer(m, top_k, num_experts, hidden, inter, 2, pre13_b != nullptr, false);
   if (workspace_bytes < p.total) {
     set_error("moe layer: workspace too small (%lld < %lld)", (long long)workspace_bytes,
               (long long)p.total);
@@ -1232,21 +1261,10 @@ extern "C" int mxfp4_moe_layer_pre(const void* x, int x_dtype, int64_t m, int64_
   if (m == 0) return MXFP4_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
   uint8_t* ws = static_cast<uint8_t*>(workspace);
-  int32_t* counts = reinterpret_cast<int32_t*>(ws + p.off_counts);
-  int32_t* sorted = reinterpret_cast<int32_t*>(ws + p.off_sorted);
-  int32_t* experts = reinterpret_cast<int32_t*>(ws + p.off_experts);
-  int32_t* npp = reinterpret_cast<int32_t*>(ws + p.off_npp);
-  void* h = ws + p.off_h;
-  void* d = ws + p.off_d;
 
   // Few routes: the GEMMs find their rows from the top-k ids directly
   // (direct routing), so no routing metadata is built.
   const bool direct = p.routes <= kDirectRoutes && inter * hidden < ((int64_t)1 << 31);
-  if (!direct) {
-    rc = do_align(topk_ids, ids_dtype, p.routes, num_experts, p.block_m, sorted, experts, npp,
-                  counts, p.nchunks, st);
-    if (rc) return rc;
-  }
 
   // gate_up with the fused SiLU*mul epilogue: h[r, :inter]
   GemmArgs g = {};
@@ -1259,41 +1277,19 @@ extern "C" int mxfp4_moe_layer_pre(const void* x, int x_dtype, int64_t m, int64_
   g.b_e = 2 * inter * (hidden / 2);
   g.bs_n = hidden / 32;
   g.bs_e = 2 * inter * (hidden / 32);
-  g.c = h;
   g.ldc = inter;
-  g.sorted_ids = sorted;
-  g.expert_ids = experts;
-  g.num_post_padded = npp;
-  g.m = p.max_sorted;
   g.num_valid = p.routes;
   g.n = (int32_t)inter;
   g.k = (int32_t)hidden;
   g.top_k = top_k;
-  g.block_m = p.block_m;
   g.inter = (int32_t)inter;
   g.num_experts = num_experts;
   g.pre_b = pre13_b;
   g.pre_s = pre13_s;
   g.pre_b_e = prepacked_nibble_bytes(2 * inter, hidden);
   g.pre_s_e = prepacked_scale_bytes(2 * inter, hidden);
-  if (direct) {
-    g.sorted_ids = nullptr;
-    g.expert_ids = nullptr;
-    g.num_post_padded = nullptr;
-    g.route_ids = topk_ids;
-    g.ids64 = ids_dtype == MXFP4_DT_I64;
-  }
-  rc = launch_w4a16(g, x_dtype, EPI_SILU_MUL, st);
-  if (rc) return rc;
-  if (direct && top_k <= 16) {
-    // down with the route weight and the top-k sum in one kernel
-    return launch_moe_down_topk(h, w2, s2, topk_weights, topk_ids, ids_dtype == MXFP4_DT_I64, m,
-                                top_k, hidden, inter, num_experts, out, x_dtype, st);
-  }
-
   // down with the route weight: d[r, :hidden]
   GemmArgs g2 = g;
-  g2.a = h;
   g2.a_rows = p.routes;
   g2.lda = inter;
   g2.b = w2;
@@ -1302,7 +1298,6 @@ extern "C" int mxfp4_moe_layer_pre(const void* x, int x_dtype, int64_t m, int64_
   g2.b_e = hidden * (inter / 2);
   g2.bs_n = inter / 32;
   g2.bs_e = hidden * (inter / 32);
-  g2.c = d;
   g2.ldc = hidden;
   g2.route_w = topk_weights;
   g2.n = (int32_t)hidden;
@@ -1313,6 +1308,49 @@ extern "C" int mxfp4_moe_layer_pre(const void* x, int x_dtype, int64_t m, int64_
   g2.pre_s = pre2_s;
   g2.pre_b_e = prepacked_nibble_bytes(hidden, inter);
   g2.pre_s_e = prepacked_scale_bytes(hidden, inter);
+  if (!direct && dr_faster(p.routes, num_experts, inter, hidden, true, pre13_b != nullptr)) {
+    // both GEMMs on 64-row blocks of w4a16_dr, where its routing fits the
+    // workspace
+    const LayerPlan q = plan_layer(m, top_k, num_experts, hidden, inter, 2, pre13_b != nullptr, true);
+    g2.a = ws + q.off_h;
+    if (workspace_bytes >= q.total && dr_supported(g) && dr_supported(g2)) {
+      p = q;
+      g.dr = g2.dr = 1;
+    }
+  }
+  int32_t* counts = reinterpret_cast<int32_t*>(ws + p.off_counts);
+  int32_t* sorted = reinterpret_cast<int32_t*>(ws + p.off_sorted);
+  int32_t* experts = reinterpret_cast<int32_t*>(ws + p.off_experts);
+  int32_t* npp = reinterpret_cast<int32_t*>(ws + p.off_npp);
+  void* h = ws + p.off_h;
+  void* d = ws + p.off_d;
+  if (!direct) {
+    rc = do_align(topk_ids, ids_dtype, p.routes, num_experts, p.block_m, sorted, experts, npp,
+                  counts, p.nchunks, st);
+    if (rc) return rc;
+  }
+  g.c = h;
+  g2.a = h;
+  g2.c = d;
+  for (GemmArgs* q : {&g, &g2}) {
+    q->m = p.max_sorted;
+    q->block_m = p.block_m;
+    if (direct) {
+      q->route_ids = topk_ids;
+      q->ids64 = ids_dtype == MXFP4_DT_I64;
+    } else {
+      q->sorted_ids = sorted;
+      q->expert_ids = experts;
+      q->num_post_padded = npp;
+    }
+  }
+  rc = launch_w4a16(g, x_dtype, EPI_SILU_MUL, st);
+  if (rc) return rc;
+  if (direct && top_k <= 16) {
+    // down with the route weight and the top-k sum in one kernel
+    return launch_moe_down_topk(h, w2, s2, topk_weights, topk_ids, ids_dtype == MXFP4_DT_I64, m,
+                                top_k, hidden, inter, num_experts, out, x_dtype, st);
+  }
   rc = launch_w4a16(g2, x_dtype, EPI_STORE, st);
   if (rc) return rc;
 
@@ -1397,6 +1435,7 @@ extern "C" int mxfp4_moe_layer_noalloc(const void* x, int x_dtype, int64_t m, in
   int64_t need = 0;
   int rc = mxfp4_moe_layer_workspace_size(m, top_k, num_experts, hidden, inter, &need);
   if (rc) return rc;
+  need = layer_bytes(m, top_k, num_experts, hidden, inter);
   if (need > kNoAllocScratchBytes) {
     set_error("moe layer (no-alloc): %lld tokens x top-%d need a %lld-byte workspace, above the "
               "%lld bytes of the fixed scratch; use mxfp4_moe_layer with a workspace",
