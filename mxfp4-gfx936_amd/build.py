@@ -4,7 +4,9 @@
 hipcc (in parallel, objects under ``_build/``) and links
 ``mxfp4_amd/libmxfp4_gfx950.so`` next to the Python package that loads it,
 and ``mxfp4_amd/libmxfp4_probe.so`` (``csrc/probe/``: a plain HBM read that
-bench.py times as the floor of the decode kernels; not part of the library).
+bench.py times as the floor of the decode kernels; not part of the library),
+and with the host compiler ``mxfp4_amd/_host.so`` (``host/``: the operators'
+plain calls, against the installed torch).
 
 Flags: ``-O3`` for gfx950 only; packed-FP32 instruction selection is turned
 off (``-Xclang -target-feature -Xclang -packed-fp32-ops``); denormals are
@@ -29,6 +31,10 @@ LIB = os.path.join(HERE, "mxfp4_amd", "libmxfp4_gfx950.so")
 # measurement aid for bench.py (a plain HBM read), kept out of the library
 PROBE_SRC = os.path.join(CSRC, "probe", "read_floor.hip")
 PROBE_LIB = os.path.join(HERE, "mxfp4_amd", "libmxfp4_probe.so")
+# the operators' plain calls in native code (torch's C++ interface)
+HOST_SRC = os.path.join(HERE, "host", "mxfp4_host.cpp")
+HOST_LIB = os.path.join(HERE, "mxfp4_amd", "_host.so")
+CXX = os.environ.get("CXX", "g++")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
@@ -61,6 +67,30 @@ def _compile(src: str, verbose: bool) -> str:
     return obj
 
 
+def _build_host(verbose: bool) -> None:
+    """The CPython module ``mxfp4_amd/_host.so`` against the installed torch."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    root = os.path.dirname(torch.__file__)
+    libs = os.path.join(root, "lib")
+    incs = [*cpp_extension.include_paths(), os.path.join(os.path.dirname(os.path.dirname(HIPCC)),
+                                                         "include"),
+            sysconfig.get_paths()["include"], INCLUDE]
+    tmp = HOST_LIB + ".tmp"
+    cmd = [CXX, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *[f"-isystem{i}" for i in incs], HOST_SRC, f"-L{libs}", "-ltorch_python", "-ltorch",
+           "-ltorch_cpu", "-lc10", "-lc10_hip", f"-Wl,-rpath,{libs}", "-o", tmp]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"{CXX} failed for {HOST_SRC}:\n{res.stdout}{res.stderr}")
+    os.replace(tmp, HOST_LIB)
+
+
 def build(verbose: bool = False) -> str:
     """Compile all HIP sources and link the shared library; returns its path."""
     os.makedirs(GEN_DIR, exist_ok=True)
@@ -70,9 +100,11 @@ def build(verbose: bool = False) -> str:
     sources = sorted(glob.glob(os.path.join(CSRC, "*.hip")))
     if not sources:
         raise RuntimeError(f"no HIP sources under {CSRC}")
-    workers = min(len(sources), max(1, min(8, os.cpu_count() or 1)))
+    workers = min(len(sources) + 1, max(1, min(8, os.cpu_count() or 1)))
     with cf.ThreadPoolExecutor(workers) as ex:
+        host = ex.submit(_build_host, verbose)
         objs = list(ex.map(lambda s: _compile(s, verbose), sources))
+        host.result()
     tmp = LIB + ".tmp"
     cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp]
     if verbose:

@@ -101,6 +101,39 @@ def load():
     return _lib
 
 
+# the entry points the native call paths use, in their order (host/mxfp4_host.cpp)
+_HOST_ENTRIES = (
+    "mxfp4_linear_w4a16_pre", "mxfp4_linear_w4a16_workspace_size", "mxfp4_moe_layer_pre",
+    "mxfp4_moe_layer_workspace_size", "mxfp4_fused_moe_pre", "mxfp4_fused_moe_workspace_size",
+    "mxfp4_moe_gemm_pre", "mxfp4_moe_align", "mxfp4_moe_align_sizes", "mxfp4_moe_route",
+    "mxfp4_quant", "mxfp4_linear_w4a4",
+)
+_host = None
+
+
+def host():
+    """The module with the operators' plain calls in native code, bound to the
+    loaded library (once); RuntimeError if it was not built.  Its functions
+    return None for a call that is not plain: the caller then runs its general
+    path, which also raises the argument errors.  None while the library
+    itself is missing (the general path says so, after those errors)."""
+    global _host
+    if _host is None:
+        if not os.path.exists(LIB_PATH):
+            return None
+        lib = load()
+        try:
+            from . import _host as mod
+        except ImportError as e:
+            raise RuntimeError(
+                f"mxfp4_amd: the native call paths (_host.so) are missing or do not fit this "
+                f"torch ({e}); build them with `python mxfp4-gfx936_amd/build.py`") from e
+        with _lock:
+            mod.bind(check, *[ctypes.cast(getattr(lib, n), _P).value for n in _HOST_ENTRIES])
+            _host = mod
+    return _host
+
+
 _ERRORS = {
     ERR_TYPE: TypeError,
     ERR_VALUE: ValueError,

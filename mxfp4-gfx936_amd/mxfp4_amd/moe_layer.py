@@ -54,6 +54,11 @@ def moe_layer(
     """
     if activation != "silu":
         raise NotImplementedError(f"the gfx936 MXFP4 adapter supports silu, got {activation}")
+    host = _lib.host()
+    out = host and host.moe_layer(x, w13, w13_scale, w2, w2_scale, topk_weights, topk_ids,
+                                  prepacked13, prepacked2)
+    if out is not None:
+        return out
     if x.dtype not in (torch.bfloat16, torch.float16):
         raise TypeError(f"x must be fp16 or bf16, got {x.dtype}")
     for t, name in ((w13, "w13"), (w13_scale, "w13_scale"), (w2, "w2"), (w2_scale, "w2_scale")):
@@ -132,6 +137,11 @@ def route_topk(router_logits: torch.Tensor, top_k: int, renormalize: bool = True
     top_k <= min(E, 64)."""
     if ids_dtype not in (torch.int32, torch.int64):
         raise TypeError(f"topk_ids dtype must be int32 or int64, got {ids_dtype}")
+    host = _lib.host()
+    out = host and host.route_topk(router_logits, top_k, bool(renormalize),
+                                   ids_dtype == torch.int32)
+    if out is not None:
+        return out
     if router_logits.dim() < 1:
         raise ValueError("router_logits needs an expert dimension")
     num_experts = router_logits.shape[-1]

@@ -37,7 +37,7 @@ import torch
 
 from . import _lib
 from .moe_op_mxfp4_soft import _FP8_DTYPES, _moe_gemm_launch, _prepare_moe_operands
-from .prepack import lookup_prepacked
+from .prepack import any_registered, lookup_prepacked
 
 _COMPUTE_NAMES = {
     torch.bfloat16: ("bfloat16", "bf16"),
@@ -78,6 +78,13 @@ def fused_moe_mxfp4(
     """aiter:367-472 semantics on gfx950 (see the module docstring)."""
     if swizzle_mx_a or swizzle_mx_b:
         raise NotImplementedError("swizzled MX scales are not supported by the gfx950 backend")
+    if (type(config) is dict and (compute_type is None or compute_type is getattr(C, "dtype", 0))
+            and not any_registered()):
+        host = _lib.host()
+        if host and host.routed(A, B, C, A_scale, B_scale, A_mx_scale, B_mx_scale, topk_weights,
+                                topk_ids, mul_routed_weight, top_k, sorted_token_ids, expert_ids,
+                                num_tokens_post_padded, config.get("BLOCK_SIZE_M")):
+            return
     # aiter:412-424
     assert topk_weights.stride(1) == 1
     assert sorted_token_ids.stride(0) == 1

@@ -24,12 +24,12 @@ import torch
 
 try:
     from . import _lib
-    from .prepack import PrepackedWeights, check_prepacked, lookup_prepacked
+    from .prepack import PrepackedWeights, any_registered, check_prepacked, lookup_prepacked
 except ImportError:  # loaded by file path, outside its package
     sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
     from mxfp4_amd import _lib  # type: ignore[no-redef]
     from mxfp4_amd.prepack import (  # type: ignore[no-redef]
-        PrepackedWeights, check_prepacked, lookup_prepacked)
+        PrepackedWeights, any_registered, check_prepacked, lookup_prepacked)
 
 # soft:12-29 (OCP E2M1 code -> value; bit 3 is the sign)
 _MXFP4_E2M1_VALUES = (
@@ -168,6 +168,11 @@ def linear_mxfp4_soft(
     a current copy recorded with ``prepack.register_prepacked(packed,
     block_scales)`` is used.
     """
+    if prepacked is not None or not any_registered():
+        host = _lib.host()
+        out = host and host.linear(x, packed, block_scales, bias, prepacked)
+        if out is not None:
+            return out
     if x.dtype not in (torch.float16, torch.bfloat16):
         raise TypeError(f"x must be fp16 or bf16, got {x.dtype}")
     if packed.dtype != torch.uint8 or block_scales.dtype != torch.uint8:
@@ -220,6 +225,10 @@ def make_routing_device(topk_ids: torch.Tensor, num_experts: int, block_m: int):
     sync.  Returns (sorted_ids, expert_ids, num_tokens_post_padded), the first
     two sized to their capacity; entries at or beyond
     ``num_tokens_post_padded[0]`` (resp. its block count) are unused."""
+    host = _lib.host()
+    out = host and host.align(topk_ids, num_experts, block_m)
+    if out is not None:
+        return out
     device = _lib.require_device(topk_ids)
     lib = _lib.load()
     ids = topk_ids.reshape(-1)
@@ -387,6 +396,11 @@ def fused_moe_mxfp4_soft(
     """
     if swizzle_mx_a or swizzle_mx_b:
         raise NotImplementedError("the gfx936 software fallback does not support swizzled scales")
+    if not any_registered():
+        host = _lib.host()
+        if host and host.soft(A, B, C, A_scale, B_scale, A_mx_scale, B_mx_scale, topk_weights,
+                              topk_ids, mul_routed_weight, top_k):
+            return
     if topk_ids.shape != topk_weights.shape or topk_ids.shape[1] != top_k:
         raise ValueError("top-k ids and weights must have matching (M, top_k) shapes")
     if B.dtype != torch.uint8 or B_mx_scale is None:

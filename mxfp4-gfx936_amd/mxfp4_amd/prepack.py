@@ -184,6 +184,11 @@ def unregister_prepacked(packed: torch.Tensor) -> None:
         _REGISTRY.pop(packed.data_ptr(), None)
 
 
+def any_registered() -> bool:
+    """Whether any copy is registered (then the operators look theirs up)."""
+    return bool(_REGISTRY)
+
+
 def _dims(packed: torch.Tensor):
     """(experts, rows, K) of dense [N, K/2] or expert [E, N, K/2] weights."""
     if packed.ndim == 2:

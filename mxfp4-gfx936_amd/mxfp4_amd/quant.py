@@ -24,12 +24,18 @@ from . import _lib
 
 _MODES = {"ties_away": _lib.QUANT_TIES_AWAY, "rne": _lib.QUANT_RNE}
 
+_OUT_CODES = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
+
 
 def dynamic_mxfp4_quant(x: torch.Tensor, mode: str = "ties_away"):
     """Quantize the last dimension of ``x`` in blocks of 32; returns
     (packed uint8 [..., K/2], scales uint8 [..., K/32])."""
     if mode not in _MODES:
         raise ValueError(f"unknown quantizer mode {mode!r}")
+    host = _lib.host()
+    out = host and host.quant(x, _MODES[mode])
+    if out is not None:
+        return out
     if x.dtype not in (torch.bfloat16, torch.float16, torch.float32):
         raise TypeError(f"x must be bf16, fp16 or fp32, got {x.dtype}")
     k = x.shape[-1]
@@ -55,6 +61,10 @@ def linear_mxfp4_w4a4(a_packed: torch.Tensor, a_scales: torch.Tensor, w_packed: 
                       w_scales: torch.Tensor, out_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
     """out [M, N] = dequant(a) . dequant(w)^T with FP32 accumulation, rounded
     once to ``out_dtype`` (bf16, fp16 or fp32)."""
+    host = _lib.host()
+    out = host and host.w4a4(a_packed, a_scales, w_packed, w_scales, _OUT_CODES.get(out_dtype, -1))
+    if out is not None:
+        return out
     for t, name in ((a_packed, "a_packed"), (a_scales, "a_scales"), (w_packed, "w_packed"),
                     (w_scales, "w_scales")):
         if t.dtype != torch.uint8:
