@@ -178,6 +178,11 @@ __device__ __forceinline__ void dr_body(const GemmArgs& g, const DrTile& t) {
     static_for<0, UP>([&](auto xx) {
       constexpr int x = decltype(xx)::value;
       const int u = p * UP + x;
+      // an odd last unit: nothing past K (its weights read as zero codes, but
+      // the scale bytes there are the next row's, and 0 x 255 is NaN)
+      if constexpr (x > 0) {
+        if (u >= nu) return;
+      }
       uint32_t sd[FN];
       // A(u) has landed (only the piece issued after it may be in flight),
       // and this wave's reads of stage u - 1, whose buffer the next loads

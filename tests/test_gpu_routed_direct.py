@@ -70,6 +70,30 @@ def test_routed_blocks(n, k, block_m, a_dtype, c_dtype):
     assert torch.equal(masked[keep], direct[keep]) and not masked[~keep].any()
 
 
+# scale byte 255 (NaN) in every other row, an odd number of 128-deep units: the
+# rows beside it stay finite (no scale byte past a row's own is applied)
+@pytest.mark.parametrize("k", [128, 384, 640])
+@pytest.mark.parametrize("n", [64, 200])
+def test_nan_scales_stay_in_their_row(n, k):
+    e = len(COUNTS)
+    ids = _routes(n + k)
+    m = ids.shape[0]
+    wp, ws = rand_mxfp4(np.random.default_rng(k), (e, n), k)
+    ws[:, 1::2, 0] = 255
+    a = cuda(rand_act(k, (m, k)))
+    srt, exp_, npp = (cuda(t) for t in O.make_routing(ids, block_m=64, num_experts=e))
+    one, ones = torch.ones(1, device="cuda"), torch.ones(e, device="cuda")
+    outs = []
+    for scales in (cuda(ws), _shifted(cuda(ws))):
+        C = torch.full((m, 1, n), 3.0, dtype=torch.bfloat16, device="cuda")
+        mx.fused_moe_mxfp4(a, cuda(wp), C, one, ones, None, scales,
+                           torch.ones((m, 1), device="cuda"), cuda(ids), srt, exp_, npp, False, 1,
+                           False, False, {"BLOCK_SIZE_M": 64}, C.dtype)
+        outs.append(C)
+    assert torch.isnan(outs[0][..., 1::2]).all() and torch.isfinite(outs[0][..., ::2]).all()
+    assert torch.equal(outs[0].nan_to_num(7.0), outs[1].nan_to_num(7.0))
+
+
 # soft op: the safe call's own routing, with dropped ids (zero rows)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,e,top_k,n,k", [(40, 16, 4, 136, 640), (300, 8, 2, 1024, 1408),
