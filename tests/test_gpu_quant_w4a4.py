@@ -68,6 +68,23 @@ def test_quant_rne_encoder_path_matches_scalar_path(dtype):
     assert np.array_equal(sa[cuda(finite)].cpu().numpy(), rs)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,k", [(1, 32), (1, 96), (3, 672), (64, 32), (65, 32), (127, 4064)])
+def test_quant_rne_contiguous_and_strided_rows(rows, k, dtype):
+    # contiguous rows run as one list of blocks (remainders of its workgroup's
+    # 64), rows with a gap by row index; whole bytes, so exact in both
+    g = torch.Generator().manual_seed(31 * rows + k)
+    x = torch.randn((rows, k), generator=g) * torch.exp2(
+        torch.randint(-8, 8, (rows, 1), generator=g).float())
+    x = x.to(dtype)
+    rp, rs = c_oracle.quant(x.float().numpy(), "rne")
+    gap = torch.zeros((rows, k + 8), dtype=dtype)
+    gap[:, :k] = x
+    for v in (cuda(x), cuda(gap)[:, :k]):
+        p, s = mx.dynamic_mxfp4_quant(v, mode="rne")
+        assert np.array_equal(p.cpu().numpy(), rp) and np.array_equal(s.cpu().numpy(), rs)
+
+
 def test_quant_golden_fixture():
     g = np.load(os.path.join(GOLDEN, "small_cases.npz"))
     x = cuda(g["quant_x"])
