@@ -338,8 +338,10 @@ PyObject* routed(PyObject*, PyObject* const* a, Py_ssize_t) {
   const at::Tensor *srt = c.take(a[11]), *exp = c.take(a[12]), *npp = c.take(a[13]);
   const int64_t bm = whole(a[14]);
   if (!c.ok || srt->scalar_type() != at::kInt || exp->scalar_type() != at::kInt ||
-      npp->scalar_type() != at::kInt || npp->numel() != 1 || bm < 16 || bm % 16 ||
-      bm > 0x7FFFFFFF || srt->dim() != 1 || srt->numel() == 0 || srt->numel() % bm ||
+      npp->scalar_type() != at::kInt || npp->numel() != 1 ||
+      // asserted by the general path, also of a dimension of size 1
+      r.tw->stride(1) != 1 || srt->dim() != 1 || srt->stride(0) != 1 || bm < 16 || bm % 16 ||
+      bm > 0x7FFFFFFF || srt->numel() == 0 || srt->numel() % bm ||
       exp->numel() * bm < srt->numel())
     return none();
   int rc = 0;

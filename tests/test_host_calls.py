@@ -174,3 +174,19 @@ def test_calls_that_are_not_plain(monkeypatch):
     mx.register_prepacked(w2, s2)
     assert torch.equal(mx.linear_mxfp4_soft(x, w2, s2), mx.linear_mxfp4_soft(x, w, s))
     mx.unregister_prepacked(w2)
+
+
+@pytest.mark.gpu
+def test_asserted_strides_of_size_one_dimensions():
+    # contiguous tensors all the same, as a dimension of size 1 has any stride
+    w13, s13 = _weights(np.random.default_rng(11), (4, 64), 128, cuda)
+    a = cuda(rand_act(6, (16, 128)))
+    ids = cuda(torch.arange(16).remainder(4).view(16, 1))
+    tw = torch.ones((16, 1), device="cuda").as_strided((16, 1), (1, 5))
+    assert tw.is_contiguous() and tw.stride(1) == 5
+    srt, exp_, npp = mx.make_routing_device(ids, 4, 16)
+    C = torch.zeros((16, 1, 64), dtype=torch.bfloat16, device="cuda")
+    one, ones = torch.ones(1, device="cuda"), torch.ones(4, device="cuda")
+    with pytest.raises(AssertionError):
+        mx.fused_moe_mxfp4(a, w13, C, one, ones, None, s13, tw, ids, srt, exp_, npp, True, 1,
+                           False, False, {"BLOCK_SIZE_M": 16}, C.dtype)
