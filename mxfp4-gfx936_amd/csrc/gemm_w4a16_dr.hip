@@ -476,7 +476,12 @@ bool dr_faster(int64_t routes, int64_t experts, int64_t n, int64_t k, bool silu,
     // too (E=32 top-4 layer, 128 / 256 routes per expert 94.1 -> 72.7 /
     // 115.6 vs 124.3) unless even their 128-row blocks leave CUs idle (E=8
     // top-2, I=1408, 256 routes per expert 93.7 -> 69.7).
-    if (avg <= 1.5) return false;
+    // The layer keeps them up to 2.5 while its experts fill less than half
+    // the CUs (E=64 top-6 at 2 routes per expert, H x I 2048x512 / 1024x1408 /
+    // 4096x512 / 2048x1024 35.2 / 44.3 / 60.9 / 57.5 vs 36.9 / 45.8 / 62.7 /
+    // 55.0; E=128 H=2048 I=768 79.6 -> 75.0; E=64 at 3, H=4096 I=1024 108.1 ->
+    // 96.5).
+    if (avg <= (silu && 2 * std::min(routes, experts) < cus ? 2.5 : 1.5)) return false;
     if (avg <= ((small || k < 2048) ? 128.0 : 80.0)) return true;
     return dr_blocks(routes, experts, 128) * nbn < cus;
   }
