@@ -28,6 +28,7 @@
 
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 
 #include "mxfp4_gfx950.h"
 
@@ -51,6 +52,17 @@ PyObject* g_check = nullptr;  // Python: raises the exception of a status
 PyObject *s_nibbles, *s_scales, *s_experts, *s_rows, *s_k, *s_source;
 
 PyObject* none() { Py_RETURN_NONE; }
+
+// f(a...) without the GIL.  The arguments are the caller's, read while it holds
+// the GIL: data_ptr() may allocate (a copy-on-write storage) and throw, and an
+// exception must not pass the point where the thread state is away.
+template <typename... P>
+int run(int (*f)(P...), std::common_type_t<P>... a) {
+  PyThreadState* state = PyEval_SaveThread();
+  const int rc = f(a...);
+  PyEval_RestoreThread(state);
+  return rc;
+}
 
 // The status' exception, or `ok` (a new reference, dropped on an error).
 PyObject* finish(int rc, PyObject* ok) {
@@ -202,11 +214,9 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t) {
   shape.back() = n;
   at::Tensor out = at::empty(shape, x->options()), ws;
   if (ws_bytes) ws = bytes(*x, ws_bytes);
-  Py_BEGIN_ALLOW_THREADS
-  rc = lib.linear(x->data_ptr(), code(x->scalar_type()), m, k, k, data<uint8_t>(w),
-                  data<uint8_t>(s), pre.nibbles, pre.scales, n, b ? b->data_ptr() : nullptr,
-                  out.data_ptr(), ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, c.stream());
-  Py_END_ALLOW_THREADS
+  rc = run(lib.linear, x->data_ptr(), code(x->scalar_type()), m, k, k, data<uint8_t>(w),
+           data<uint8_t>(s), pre.nibbles, pre.scales, n, b ? b->data_ptr() : nullptr,
+           out.data_ptr(), ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, c.stream());
   return finish(rc, rc ? nullptr : THPVariable_Wrap(std::move(out)));
   END_HANDLE_TH_ERRORS
 }
@@ -243,13 +253,10 @@ PyObject* moe_layer(PyObject*, PyObject* const* a, Py_ssize_t) {
   int rc = lib.layer_ws(m, top_k, (int)e, hidden, inter, &ws_bytes);
   if (rc) return finish(rc, nullptr);
   at::Tensor out = at::empty({m, hidden}, x->options()), ws = bytes(*x, ws_bytes);
-  Py_BEGIN_ALLOW_THREADS
-  rc = lib.layer(x->data_ptr(), code(x->scalar_type()), m, hidden, data<uint8_t>(w13),
-                 data<uint8_t>(s13), p13.nibbles, p13.scales, data<uint8_t>(w2), data<uint8_t>(s2),
-                 p2.nibbles, p2.scales, (int)e, inter, data<float>(tw), ids->data_ptr(),
-                 code(ids->scalar_type()), top_k, out.data_ptr(), ws.data_ptr(), ws_bytes,
-                 c.stream());
-  Py_END_ALLOW_THREADS
+  rc = run(lib.layer, x->data_ptr(), code(x->scalar_type()), m, hidden, data<uint8_t>(w13),
+           data<uint8_t>(s13), p13.nibbles, p13.scales, data<uint8_t>(w2), data<uint8_t>(s2),
+           p2.nibbles, p2.scales, (int)e, inter, data<float>(tw), ids->data_ptr(),
+           code(ids->scalar_type()), top_k, out.data_ptr(), ws.data_ptr(), ws_bytes, c.stream());
   return finish(rc, rc ? nullptr : THPVariable_Wrap(std::move(out)));
   END_HANDLE_TH_ERRORS
 }
@@ -314,13 +321,11 @@ PyObject* soft(PyObject*, PyObject* const* a, Py_ssize_t) {
   int rc = lib.fused_ws(r.m, r.top_k, r.e, act, out, &ws_bytes);
   if (rc) return finish(rc, nullptr);
   at::Tensor ws = bytes(*r.A, ws_bytes);
-  Py_BEGIN_ALLOW_THREADS
-  rc = lib.fused(r.A->data_ptr(), act, r.A->size(0), r.A->size(1), data<uint8_t>(r.amx),
-                 data<uint8_t>(r.B), data<uint8_t>(r.bmx), nullptr, nullptr, r.e, r.n, r.k,
-                 r.C->data_ptr(), out, data<float>(r.as), data<float>(r.bs), data<float>(r.tw),
-                 a[9] == Py_True ? 1 : 0, r.ids->data_ptr(), code(r.ids->scalar_type()), r.m,
-                 r.top_k, ws.data_ptr(), ws_bytes, c.stream());
-  Py_END_ALLOW_THREADS
+  rc = run(lib.fused, r.A->data_ptr(), act, r.A->size(0), r.A->size(1), data<uint8_t>(r.amx),
+           data<uint8_t>(r.B), data<uint8_t>(r.bmx), nullptr, nullptr, r.e, r.n, r.k,
+           r.C->data_ptr(), out, data<float>(r.as), data<float>(r.bs), data<float>(r.tw),
+           a[9] == Py_True ? 1 : 0, r.ids->data_ptr(), code(r.ids->scalar_type()), r.m, r.top_k,
+           ws.data_ptr(), ws_bytes, c.stream());
   Py_INCREF(Py_True);
   return finish(rc, Py_True);
   END_HANDLE_TH_ERRORS
@@ -344,15 +349,13 @@ PyObject* routed(PyObject*, PyObject* const* a, Py_ssize_t) {
       bm > 0x7FFFFFFF || srt->numel() == 0 || srt->numel() % bm ||
       exp->numel() * bm < srt->numel())
     return none();
-  int rc = 0;
-  Py_BEGIN_ALLOW_THREADS
-  rc = lib.gemm(r.A->data_ptr(), code(r.A->scalar_type()), r.A->size(0), r.A->size(1),
-                data<uint8_t>(r.amx), data<uint8_t>(r.B), data<uint8_t>(r.bmx), nullptr, nullptr,
-                r.e, r.n, r.k, r.C->data_ptr(), code(r.C->scalar_type()), r.n, data<float>(r.as),
-                data<float>(r.bs), data<float>(r.tw), a[9] == Py_True ? 1 : 0, data<int32_t>(srt),
-                data<int32_t>(exp), data<int32_t>(npp), srt->numel(), (int)bm, r.ids->numel(),
-                r.top_k, c.stream());
-  Py_END_ALLOW_THREADS
+  const int rc = run(lib.gemm, r.A->data_ptr(), code(r.A->scalar_type()), r.A->size(0),
+                     r.A->size(1), data<uint8_t>(r.amx), data<uint8_t>(r.B), data<uint8_t>(r.bmx),
+                     nullptr, nullptr, r.e, r.n, r.k, r.C->data_ptr(), code(r.C->scalar_type()),
+                     r.n, data<float>(r.as), data<float>(r.bs), data<float>(r.tw),
+                     a[9] == Py_True ? 1 : 0, data<int32_t>(srt), data<int32_t>(exp),
+                     data<int32_t>(npp), srt->numel(), (int)bm, r.ids->numel(), r.top_k,
+                     c.stream());
   Py_INCREF(Py_True);
   return finish(rc, Py_True);
   END_HANDLE_TH_ERRORS
@@ -374,11 +377,9 @@ PyObject* align(PyObject*, PyObject* const* a, Py_ssize_t) {
   const auto opt = ids->options().dtype(at::kInt);
   at::Tensor sorted = at::empty({ms}, opt), experts = at::empty({mb}, opt),
              npp = at::empty({1}, opt), ws = bytes(*ids, wsb > 4 ? wsb : 4);
-  Py_BEGIN_ALLOW_THREADS
-  rc = lib.align(ids->data_ptr(), code(ids->scalar_type()), n, (int)e, (int)bm,
-                 data<int32_t>(&sorted), data<int32_t>(&experts), data<int32_t>(&npp),
-                 ws.data_ptr(), wsb, c.stream());
-  Py_END_ALLOW_THREADS
+  rc = run(lib.align, ids->data_ptr(), code(ids->scalar_type()), n, (int)e, (int)bm,
+           data<int32_t>(&sorted), data<int32_t>(&experts), data<int32_t>(&npp), ws.data_ptr(), wsb,
+           c.stream());
   if (rc) return finish(rc, nullptr);
   return Py_BuildValue("(NNN)", THPVariable_Wrap(std::move(sorted)),
                        THPVariable_Wrap(std::move(experts)), THPVariable_Wrap(std::move(npp)));
@@ -401,11 +402,8 @@ PyObject* route_topk(PyObject*, PyObject* const* a, Py_ssize_t) {
   shape.back() = top;
   at::Tensor w = at::empty(shape, l->options()), ids = at::empty(shape, l->options().dtype(type));
   const int renorm = PyObject_IsTrue(a[2]) ? 1 : 0;
-  int rc = 0;
-  Py_BEGIN_ALLOW_THREADS
-  rc = lib.route(data<float>(l), l->numel() / e, (int)e, e, (int)top, renorm, data<float>(&w),
-                 ids.data_ptr(), code(type), c.stream());
-  Py_END_ALLOW_THREADS
+  const int rc = run(lib.route, data<float>(l), l->numel() / e, (int)e, e, (int)top, renorm,
+                     data<float>(&w), ids.data_ptr(), code(type), c.stream());
   if (rc) return finish(rc, nullptr);
   return Py_BuildValue("(NN)", THPVariable_Wrap(std::move(w)), THPVariable_Wrap(std::move(ids)));
   END_HANDLE_TH_ERRORS
@@ -428,11 +426,8 @@ PyObject* quant(PyObject*, PyObject* const* a, Py_ssize_t) {
   at::Tensor packed = at::empty(shape, opt);
   shape.back() = k / 32;
   at::Tensor scales = at::empty(shape, opt);
-  int rc = 0;
-  Py_BEGIN_ALLOW_THREADS
-  rc = lib.quant(x->data_ptr(), code(x->scalar_type()), x->numel() / k, k, k, mode,
-                 data<uint8_t>(&packed), data<uint8_t>(&scales), c.stream());
-  Py_END_ALLOW_THREADS
+  const int rc = run(lib.quant, x->data_ptr(), code(x->scalar_type()), x->numel() / k, k, k, mode,
+                     data<uint8_t>(&packed), data<uint8_t>(&scales), c.stream());
   if (rc) return finish(rc, nullptr);
   return Py_BuildValue("(NN)", THPVariable_Wrap(std::move(packed)),
                        THPVariable_Wrap(std::move(scales)));
@@ -457,11 +452,8 @@ PyObject* w4a4(PyObject*, PyObject* const* a, Py_ssize_t) {
   if (t < 0 || t > 2) return none();
   const auto type = t == 0 ? at::kBFloat16 : (t == 1 ? at::kHalf : at::kFloat);
   at::Tensor out = at::empty({m, n}, x->options().dtype(type));
-  int rc = 0;
-  Py_BEGIN_ALLOW_THREADS
-  rc = lib.w4a4(data<uint8_t>(x), data<uint8_t>(xs), m, k, data<uint8_t>(w), data<uint8_t>(ws), n,
-                out.data_ptr(), code(type), c.stream());
-  Py_END_ALLOW_THREADS
+  const int rc = run(lib.w4a4, data<uint8_t>(x), data<uint8_t>(xs), m, k, data<uint8_t>(w),
+                     data<uint8_t>(ws), n, out.data_ptr(), code(type), c.stream());
   return finish(rc, rc ? nullptr : THPVariable_Wrap(std::move(out)));
   END_HANDLE_TH_ERRORS
 }

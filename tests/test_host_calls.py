@@ -190,3 +190,28 @@ def test_asserted_strides_of_size_one_dimensions():
     with pytest.raises(AssertionError):
         mx.fused_moe_mxfp4(a, w13, C, one, ones, None, s13, tw, ids, srt, exp_, npp, True, 1,
                            False, False, {"BLOCK_SIZE_M": 16}, C.dtype)
+
+
+@pytest.mark.gpu
+def test_failing_pointer_read_is_an_ordinary_exception():
+    # the read throws after the call has been found plain (as a copy-on-write
+    # storage does that cannot be copied): an exception as in the general path,
+    # with the interpreter lock held, and the next call runs
+    rng = np.random.default_rng(13)
+    w, s = _weights(rng, (64,), 256, cuda)
+    x = cuda(rand_act(8, (4, 256)))
+    bad = x.clone()
+    torch._C._set_throw_on_mutable_data_ptr(bad)
+    logits = torch.randn((4, 8), device="cuda")
+    bad_logits = logits.clone()
+    torch._C._set_throw_on_mutable_data_ptr(bad_logits)
+    for _ in range(2):
+        with pytest.raises(RuntimeError):
+            _lib.host().linear(bad, w, s, None, None)
+        with pytest.raises(RuntimeError):
+            _lib.host().quant(bad, 0)
+        with pytest.raises(RuntimeError):
+            _lib.host().route_topk(bad_logits, 2, True, False)
+    with pytest.raises(RuntimeError):
+        mx.linear_mxfp4_soft(bad, w, s)
+    assert torch.isfinite(mx.linear_mxfp4_soft(x, w, s)).all()
