@@ -29,6 +29,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <type_traits>
+#include <utility>
 
 #include "mxfp4_gfx950.h"
 
@@ -49,6 +50,7 @@ struct Library {
   decltype(&mxfp4_linear_w4a4) w4a4 = nullptr;
 } lib;
 PyObject* g_check = nullptr;  // Python: raises the exception of a status
+PyObject* g_pre = nullptr;    // the class PrepackedWeights
 PyObject *s_nibbles, *s_scales, *s_experts, *s_rows, *s_k, *s_source;
 
 PyObject* none() { Py_RETURN_NONE; }
@@ -166,6 +168,8 @@ struct Pre {
   bool read(Call& c, PyObject* o, int64_t experts, int64_t rows, int64_t k, const at::Tensor& w,
             const at::Tensor& s) {
     if (o == Py_None) return true;
+    // nothing that only has its attributes: the general path refuses that
+    if (reinterpret_cast<PyObject*>(Py_TYPE(o)) != g_pre) return false;
     bool good = is(o, s_experts, experts) && is(o, s_rows, rows) && is(o, s_k, k);
     PyObject* src = good ? PyObject_GetAttr(o, s_source) : nullptr;
     PyObject* n = src != nullptr ? PyObject_GetAttr(o, s_nibbles) : nullptr;
@@ -458,25 +462,25 @@ PyObject* w4a4(PyObject*, PyObject* const* a, Py_ssize_t) {
   END_HANDLE_TH_ERRORS
 }
 
-// bind(check, address, ...): the library's entry points, in Library's order
+// bind(check, PrepackedWeights, address, ...): the library's entry points, in Library's order
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
   constexpr Py_ssize_t kEntries = sizeof(Library) / sizeof(void*);
-  if (n != 1 + kEntries) {
+  if (n != 2 + kEntries) {
     PyErr_SetString(PyExc_TypeError, "bind: wrong number of entry points");
     return nullptr;
   }
   void* at[kEntries];
   for (Py_ssize_t i = 0; i < kEntries; ++i) {
-    at[i] = PyLong_AsVoidPtr(a[1 + i]);
+    at[i] = PyLong_AsVoidPtr(a[2 + i]);
     if (at[i] == nullptr) {
       if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "bind: null entry point");
       return nullptr;
     }
   }
   std::memcpy(static_cast<void*>(&lib), at, sizeof(lib));
-  Py_INCREF(a[0]);
-  Py_XDECREF(g_check);
-  g_check = a[0];
+  for (Py_ssize_t i = 0; i < 2; ++i) Py_INCREF(a[i]);
+  Py_XDECREF(std::exchange(g_check, a[0]));
+  Py_XDECREF(std::exchange(g_pre, a[1]));
   Py_RETURN_NONE;
 }
 

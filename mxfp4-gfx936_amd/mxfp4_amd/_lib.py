@@ -128,8 +128,10 @@ def host():
             raise RuntimeError(
                 f"mxfp4_amd: the native call paths (_host.so) are missing or do not fit this "
                 f"torch ({e}); build them with `python mxfp4-gfx936_amd/build.py`") from e
+        from .prepack import PrepackedWeights  # imports this module
         with _lock:
-            mod.bind(check, *[ctypes.cast(getattr(lib, n), _P).value for n in _HOST_ENTRIES])
+            mod.bind(check, PrepackedWeights,
+                     *[ctypes.cast(getattr(lib, n), _P).value for n in _HOST_ENTRIES])
             _host = mod
     return _host
 

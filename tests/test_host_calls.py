@@ -5,6 +5,8 @@ shapes the native code does not take."""
 
 from __future__ import annotations
 
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 import torch
@@ -215,3 +217,26 @@ def test_failing_pointer_read_is_an_ordinary_exception():
     with pytest.raises(RuntimeError):
         mx.linear_mxfp4_soft(bad, w, s)
     assert torch.isfinite(mx.linear_mxfp4_soft(x, w, s)).all()
+
+
+@pytest.mark.gpu
+def test_only_prepacked_weights_pass_as_a_copy():
+    # an object with the same attributes is refused, as by the general path
+    rng = np.random.default_rng(17)
+    w13, s13 = _weights(rng, (4, 256), 128, cuda)
+    w2, s2 = _weights(rng, (4, 128), 128, cuda)
+    x = cuda(rand_act(9, (20, 128)))
+    tw, ids = mx.route_topk(torch.randn((20, 4), device="cuda"), 2)
+
+    def like(pre):
+        return SimpleNamespace(**{f: getattr(pre, f) for f in pre.__dataclass_fields__})
+
+    pre, pre13, pre2 = (mx.prepack_w4a16(*p) for p in ((w13[0], s13[0]), (w13, s13), (w2, s2)))
+    assert _lib.host().linear(x, w13[0], s13[0], None, pre) is not None
+    assert _lib.host().linear(x, w13[0], s13[0], None, like(pre)) is None
+    with pytest.raises(TypeError):
+        mx.linear_mxfp4_soft(x, w13[0], s13[0], prepacked=like(pre))
+    mx.moe_layer(x, w13, s13, w2, s2, tw, ids, prepacked13=pre13, prepacked2=pre2)
+    for a, b in ((like(pre13), pre2), (pre13, like(pre2))):
+        with pytest.raises(TypeError):
+            mx.moe_layer(x, w13, s13, w2, s2, tw, ids, prepacked13=a, prepacked2=b)
