@@ -73,14 +73,16 @@ def _build_host(verbose: bool) -> None:
 
     import torch
     from torch.utils import cpp_extension
+    version = f"{torch.__version__} {torch.version.git_version}"  # as _lib.torch_build
     root = os.path.dirname(torch.__file__)
     libs = os.path.join(root, "lib")
     incs = [*cpp_extension.include_paths(), os.path.join(os.path.dirname(os.path.dirname(HIPCC)),
                                                          "include"),
             sysconfig.get_paths()["include"], INCLUDE]
     tmp = HOST_LIB + ".tmp"
-    cmd = [CXX, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1",
-           "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+    cmd = [CXX, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f'-DMXFP4_TORCH="{version}"',
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            *[f"-isystem{i}" for i in incs], HOST_SRC, f"-L{libs}", "-ltorch_python", "-ltorch",
            "-ltorch_cpu", "-lc10", "-lc10_hip", f"-Wl,-rpath,{libs}", "-o", tmp]
     if verbose:

@@ -33,6 +33,10 @@
 
 #include "mxfp4_gfx950.h"
 
+#ifndef MXFP4_TORCH
+#error "MXFP4_TORCH: the torch build compiled against (build.py sets it)"
+#endif
+
 namespace {
 
 struct Library {
@@ -513,5 +517,8 @@ PyMODINIT_FUNC PyInit__host(void) {
   s_rows = PyUnicode_InternFromString("rows");
   s_k = PyUnicode_InternFromString("k");
   s_source = PyUnicode_InternFromString("source");
-  return PyModule_Create(&module);
+  PyObject* m = PyModule_Create(&module);
+  // at::Tensor is read through inlined accessors: right for this torch only
+  if (m != nullptr && PyModule_AddStringConstant(m, "TORCH", MXFP4_TORCH) != 0) Py_CLEAR(m);
+  return m;
 }

@@ -9,8 +9,10 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import importlib
 import os
 import threading
+import warnings
 
 import torch
 
@@ -74,6 +76,7 @@ SIGNATURES = {
 
 _lib = None
 _lock = threading.Lock()
+_host_lock = threading.Lock()
 
 
 def load():
@@ -111,29 +114,52 @@ _HOST_ENTRIES = (
 _host = None
 
 
+def torch_build() -> str:
+    """The installed torch: version and source revision."""
+    return f"{torch.__version__} {torch.version.git_version}"
+
+
+def _load_host():
+    """The native module bound to the library, or False (with a warning) when
+    it is missing or was compiled against another torch: it reads tensors
+    through that torch's inlined accessors, so a layout that moved would be
+    misread without an error."""
+    lib = load()
+    try:
+        mod = importlib.import_module("._host", __package__)
+        built = getattr(mod, "TORCH", "of unknown version")
+        fault = (None if built == torch_build() else
+                 f"was compiled against torch {built}, installed is {torch_build()}")
+    except ImportError as e:
+        fault = f"does not load ({e})"
+    if fault is not None:
+        warnings.warn(f"mxfp4_amd: _host.so {fault}; the operators run without their native call "
+                      "paths (slower on the host; `python mxfp4-gfx936_amd/build.py` builds it)",
+                      RuntimeWarning, stacklevel=4)
+        return False
+    from .prepack import PrepackedWeights  # imports this module
+    mod.bind(check, PrepackedWeights,
+             *[ctypes.cast(getattr(lib, n), _P).value for n in _HOST_ENTRIES])
+    return mod
+
+
 def host():
     """The module with the operators' plain calls in native code, bound to the
-    loaded library (once); RuntimeError if it was not built.  Its functions
-    return None for a call that is not plain: the caller then runs its general
-    path, which also raises the argument errors.  None while the library
-    itself is missing (the general path says so, after those errors)."""
+    loaded library (once).  Its functions return None for a call that is not
+    plain: the caller then runs its general path, which also raises the
+    argument errors.  None (every call takes the general path) if the module
+    was not built or does not fit this torch, and while the library itself is
+    missing (the general path says so, after those errors)."""
     global _host
     if _host is None:
         if not os.path.exists(LIB_PATH):
             return None
-        lib = load()
-        try:
-            from . import _host as mod
-        except ImportError as e:
-            raise RuntimeError(
-                f"mxfp4_amd: the native call paths (_host.so) are missing or do not fit this "
-                f"torch ({e}); build them with `python mxfp4-gfx936_amd/build.py`") from e
-        from .prepack import PrepackedWeights  # imports this module
-        with _lock:
-            mod.bind(check, PrepackedWeights,
-                     *[ctypes.cast(getattr(lib, n), _P).value for n in _HOST_ENTRIES])
-            _host = mod
-    return _host
+        load()
+        with _host_lock:
+            if _host is None:
+                _host = False  # also when the warning is turned into an error
+                _host = _load_host()
+    return _host or None
 
 
 _ERRORS = {

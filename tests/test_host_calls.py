@@ -5,7 +5,9 @@ shapes the native code does not take."""
 
 from __future__ import annotations
 
-from types import SimpleNamespace
+import sys
+import warnings
+from types import ModuleType, SimpleNamespace
 
 import numpy as np
 import pytest
@@ -37,6 +39,27 @@ def test_cpu_tensors_and_wrong_counts_are_not_taken():
         host.linear(x, w, s)
     with pytest.raises(TypeError):
         host.bind(_lib.check)
+
+
+@pytest.mark.parametrize("fault", ["another torch", "no module", "no version"])
+def test_module_that_does_not_fit_leaves_the_general_path(fault, monkeypatch):
+    assert _lib.host().TORCH == _lib.torch_build()
+    monkeypatch.setattr(_lib, "_host", None)
+    if fault == "another torch":
+        monkeypatch.setattr(_lib, "torch_build", lambda: "2.0.0 0123abcd")
+    else:
+        monkeypatch.setitem(sys.modules, "mxfp4_amd._host",
+                            None if fault == "no module" else ModuleType("mxfp4_amd._host"))
+    with pytest.warns(RuntimeWarning, match="_host.so"):
+        assert _lib.host() is None
+    with warnings.catch_warnings():  # said once
+        warnings.simplefilter("error")
+        assert _lib.host() is None
+        # the operators go on to their own checks
+        with pytest.raises(RuntimeError, match="ROCm devices only"):
+            mx.linear_mxfp4_soft(torch.zeros((2, 128), dtype=torch.bfloat16),
+                                 torch.zeros((32, 64), dtype=torch.uint8),
+                                 torch.zeros((32, 4), dtype=torch.uint8))
 
 
 # ------------------------------------------------------------------- GPU
