@@ -193,7 +193,12 @@ __global__ __launch_bounds__(256) void align_place(const TI* __restrict__ ids, i
 // places the kOneChunk routes of chunk c and derives what it needs from the
 // ids themselves -- every workgroup counts all routes before and after its
 // chunk per expert (coalesced loads, LDS atomics) -- so no workgroup waits
-// for another and no counts pass through memory.  Then the padded exclusive
+// for another and no counts pass through memory.  The atomics of lanes with
+// the same expert run one after the other, up to 64 where most routes go to
+// one expert (the soft op of a rank that holds few of the experts counts all
+// others' routes on one), so the counts are kept kOneCopies times, one copy
+// per lane % kOneCopies on banks of its own (odd stride), both counts in one
+// word (each <= kOneLaunch < 2^16).  Then the padded exclusive
 // scan over the experts; the lanes of a wave with the same expert come from
 // ballots (one per id bit), their counts become each wave's first position
 // per expert, and every route lands at its wave's position + its rank among
@@ -202,15 +207,20 @@ __global__ __launch_bounds__(256) void align_place(const TI* __restrict__ ids, i
 // x % gridDim.x == c, and workgroup 0 the padded route count; small routings
 // launch kOneLeast workgroups for that (with one, its 8 waves walk 16
 // experts' padding each: 256 routes 7.9 us, with 16 to 64 workgroups 4.3).
-// Latency bound: one round of id loads, three barriers, one round of
-// stores.  Graph replays of the call, 128 experts, 64-row blocks, 256 / 1024
-// / 4096 / 8000 / 16384 routes: 4.3 / 4.5 / 4.9 / 5.5 / 7.3 us, against 5.7 /
-// 6.2 / 6.5 us in one workgroup (all phases on one CU) and 7.9 / 7.8 us for
-// the count and scan + place launches, which win above (32768 routes: 10.4
-// us here, where every workgroup counts every id, against 7.8).
+// Latency bound: a round of id loads per 8192 routes, three barriers, one
+// round of stores.  Graph replays of the call, 129 experts, 64-row blocks,
+// 1024 / 4096 / 8192 / 16384 routes: uniform ids 5.6 / 6.0 / 6.4 / 8.2 us,
+// 90% on one expert 5.6 / 6.1 / 7.0 / 9.0 (with one copy 5.6 / 7.8 / 10.8 /
+// 17.0, with eight 5.7 / 6.1 / 6.5 / 8.2 but 0.1 us more on uniform ids),
+// against 7.2 / 7.8 and 6.8 / 9.2 us in one workgroup up to 4096 routes (all
+// phases on one CU) and 9.4 / 9.3 and 9.5 / 9.4 us for the count and scan +
+// place launches, which win above (32768 uniform routes, where every
+// workgroup counts every id, 10.4 us against 7.8).  8 experts, 256 routes:
+// 5.2 us against 5.0 in one workgroup of 256 threads.
 constexpr int kOneChunk = 512;
 constexpr int64_t kOneLeast = 16;
 constexpr int64_t kOneLaunch = 16384;
+constexpr int kOneCopies = 4;
 
 template <typename TI>
 __global__ __launch_bounds__(kOneChunk) void align_one(const TI* __restrict__ ids, int64_t n,
@@ -223,21 +233,24 @@ __global__ __launch_bounds__(kOneChunk) void align_one(const TI* __restrict__ id
   constexpr int EPT = kMaxExperts / NT;  // experts per thread in the scan
   constexpr int B = 16;                  // id loads per thread per round trip
   __shared__ int wpos[W * kMaxExperts];  // [wave][expert]: counts, then next positions
-  // routes of earlier / later chunks; then first slot / first sentinel slot
-  __shared__ int s_pre[kMaxExperts], s_post[kMaxExperts];
+  // [copy][expert]: routes of earlier (low half) and of later chunks (high)
+  __shared__ uint32_t cnt[kOneCopies * (kMaxExperts + 1)];
+  __shared__ int s_start[kMaxExperts], s_fill[kMaxExperts];  // first slot, first sentinel slot
   __shared__ int part[W];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int c = (int)blockIdx.x, nwg = (int)gridDim.x;
   const int ne = num_experts;
+  const int stride = ne | 1;
+  uint32_t* const my_cnt = cnt + (lane % kOneCopies) * stride;
   const int64_t mine = (int64_t)c * NT + tid;
   const int eid = mine < n ? route_expert(ids[mine], ne, drop_to) : -1;
   TI v[B];
 #pragma unroll
   for (int b = 0; b < B; ++b) v[b] = (int64_t)b * NT + tid < n ? ids[b * NT + tid] : (TI)0;
   for (int i = tid; i < W * ne; i += NT) wpos[i] = 0;
-  for (int x = tid; x < ne; x += NT) s_pre[x] = s_post[x] = 0;
+  for (int i = tid; i < kOneCopies * stride; i += NT) cnt[i] = 0;
   __syncthreads();
   for (int64_t i0 = 0; i0 < n; i0 += B * NT) {
     if (i0 > 0) {
@@ -252,7 +265,7 @@ __global__ __launch_bounds__(kOneChunk) void align_one(const TI* __restrict__ id
       const int cc = (int)(i0 / NT) + b;
       if (cc == c || i0 + b * NT + tid >= n) continue;
       const int e = route_expert(v[b], ne, drop_to);
-      if (e >= 0) atomicAdd(cc < c ? &s_pre[e] : &s_post[e], 1);
+      if (e >= 0) atomicAdd(&my_cnt[e], cc < c ? 1u : 1u << 16);
     }
   }
   const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
@@ -267,13 +280,17 @@ __global__ __launch_bounds__(kOneChunk) void align_one(const TI* __restrict__ id
   __syncthreads();
   // padded exclusive scan over the experts (thread-local EPT, wave shuffles,
   // then the wave sums)
-  int tot[EPT], pad[EPT], local = 0;
+  int pre[EPT], tot[EPT], pad[EPT], local = 0;
 #pragma unroll
   for (int jj = 0; jj < EPT; ++jj) {
     const int x = tid * EPT + jj;
-    tot[jj] = 0;
+    pre[jj] = tot[jj] = 0;
     if (x < ne) {
-      tot[jj] = s_pre[x] + s_post[x];
+      uint32_t others = 0;
+#pragma unroll
+      for (int q = 0; q < kOneCopies; ++q) others += cnt[q * stride + x];
+      pre[jj] = (int)(others & 0xFFFF);
+      tot[jj] = pre[jj] + (int)(others >> 16);
 #pragma unroll
       for (int w = 0; w < W; ++w) tot[jj] += wpos[w * ne + x];
     }
@@ -294,15 +311,15 @@ __global__ __launch_bounds__(kOneChunk) void align_one(const TI* __restrict__ id
   for (int jj = 0; jj < EPT; ++jj) {
     const int x = tid * EPT + jj;
     if (x < ne) {
-      int p = start + s_pre[x];
+      int p = start + pre[jj];
 #pragma unroll
       for (int w = 0; w < W; ++w) {
         const int cw = wpos[w * ne + x];
         wpos[w * ne + x] = p;
         p += cw;
       }
-      s_pre[x] = start;
-      s_post[x] = start + tot[jj];
+      s_start[x] = start;
+      s_fill[x] = start + tot[jj];
     }
     start += pad[jj];
   }
@@ -310,7 +327,7 @@ __global__ __launch_bounds__(kOneChunk) void align_one(const TI* __restrict__ id
   __syncthreads();
   if (eid >= 0) sorted_ids[wpos[wave * ne + eid] + rank] = (int32_t)mine;
   for (int x = c + wave * nwg; x < ne; x += W * nwg) {
-    const int st = s_pre[x], fill = s_post[x];
+    const int st = s_start[x], fill = s_fill[x];
     const int blocks = (fill - st + block_m - 1) / block_m;
     for (int i = lane; i < blocks; i += 64) expert_ids[st / block_m + i] = x;
     for (int q = fill + lane; q < st + blocks * block_m; q += 64) sorted_ids[q] = (int32_t)n;

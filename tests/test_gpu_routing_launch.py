@@ -41,3 +41,16 @@ def test_one_launch_routing_all_dropped():
     ids = torch.full((70, 8), -1)
     _, _, npp = mx.make_routing(cuda(ids), block_m=64, num_experts=16)
     assert int(npp[0]) == 0
+
+
+# every route on one expert: the largest counts before and after a chunk, on
+# one word of each of the kernel's count copies
+@pytest.mark.parametrize("num_experts", [1, 2, 129, 1024])
+@pytest.mark.parametrize("routes", [512, 16384])
+def test_one_launch_routing_single_expert(routes, num_experts):
+    for expert in {0, num_experts - 1}:
+        ids = torch.full((routes, 1), expert)
+        srt, exp_, npp = mx.make_routing(cuda(ids), block_m=64, num_experts=num_experts)
+        assert int(npp[0]) == routes
+        assert np.array_equal(srt[:routes].cpu().numpy(), np.arange(routes))
+        assert (exp_[:routes // 64] == expert).all()
