@@ -225,7 +225,8 @@ int pf_choose(const GemmArgs& g, int epi);
 int launch_w4a16_pf(const GemmArgs& g, int dtype, int epi, int cfg, hipStream_t st);
 // Routed GEMM with the weights straight into registers (gemm_w4a16_dr.hip).
 bool dr_supported(const GemmArgs& g);
-bool dr_faster(int64_t routes, int64_t experts, int64_t n, int64_t k, bool silu, bool prepacked);
+bool dr_faster(int64_t routes, int64_t experts, int64_t n, int64_t k, bool silu, bool prepacked,
+               int block_m, int64_t cus);
 int launch_w4a16_dr(const GemmArgs& g, int dtype, int epi, hipStream_t st);
 // Split-K plan for a dense plain-epilogue GEMM whose tiles would not fill
 // the chip: the tile configuration and slice count (1 = no split).

@@ -39,6 +39,7 @@
 // No spills are allowed here: scratch accesses count in vmcnt out of order
 // with the loads, and the stage waits count loads.
 #include <algorithm>
+#include <cmath>
 
 #include "gemm.h"
 #include "silu.h"
@@ -437,11 +438,30 @@ int launch_layout(const GemmArgs& g, bool wide, hipStream_t st) {
   return launch_shape<T, EPI, false>(g, wide, st);
 }
 
-// Expert blocks of `rows` rows that the routes fill: at least one per busy
-// expert, and half a block of padding each beyond that.
+// Expert blocks of `rows` rows that the routes fill when their experts are
+// drawn alike: an expert with `avg` routes on average, deviation sqrt(avg),
+// has a block beyond j * rows if it has more routes than that.
 int64_t dr_blocks(int64_t routes, int64_t experts, int64_t rows) {
   const int64_t busy = std::min(routes, experts);
-  return std::max(busy, routes / rows + busy / 2);
+  if (busy <= 0) return 0;
+  const double avg = (double)routes / (double)busy, dev = std::sqrt(avg), r = (double)rows;
+  const double sure = std::floor(std::max(0.0, avg - 2.0 * dev) / r);  // P = 1 up to here
+  double per = 1.0 + sure;
+  for (double over = avg - (sure + 1.0) * r; over > -2.0 * dev; over -= r)
+    per += 0.5 + over / (4.0 * dev);
+  return (int64_t)((double)busy * per);
+}
+
+// 256-column tiles instead of 128-column ones: once there are 1.6 for every
+// CU (us of the call on 128-column tiles against 256-column ones, E x K x N at
+// routes per expert: 64x2048x1536 at 48, 384 wide tiles, 36.2 against 39.0;
+// 32x2048x1536 at 96, 384, 32.5 against 36.6; 64x2048x1536 on 32-row blocks at
+// 24, 417, 1.09 times as fast on wide ones; 32x2048x1536 at 128, 480, 45.9
+// against 37.5; 64x4096x1024 at 80, 497, 86.7 against 73.0; 128x2048x1536 at
+// 16, 768, 57.0 against 52.1).
+bool dr_wide(int64_t routes, int64_t experts, int64_t n, bool silu, int rows, int64_t cus) {
+  const int out = silu ? 128 : 256;
+  return 10 * dr_blocks(routes, experts, rows) * ((n + out - 1) / out) >= 16 * cus;
 }
 
 }  // namespace
@@ -456,57 +476,97 @@ bool dr_supported(const GemmArgs& g) {
   return pf_supported(g, 2);
 }
 
-// Whether the routed GEMM `g` (n output columns, `routes` routes over its
-// experts, block size still open) runs faster here, on 64-row blocks, than
-// on the prefill tiles; us of the whole call, prefill tiles -> this.
-bool dr_faster(int64_t routes, int64_t experts, int64_t n, int64_t k, bool silu, bool prepacked) {
+// Whether the routed GEMM (n output columns, K = k, `routes` routes over its
+// experts) runs faster here, on 64-row blocks (32-row ones of a caller), than
+// on the kernels its blocks of `block_m` rows (a caller's, or the ones the
+// call would plan without this kernel) take otherwise: the 16-row decode
+// kernels, or the prefill tiles.  Figures: us of the whole call in graph
+// replays over weights that do not fit the MALL, E x K x N at routes per
+// expert, those kernels -> this where it is taken, "vs" where it is not; top-k
+// of softmaxed N(0, 1) logits, "skewed" with an N(0, 1) bias per expert.
+bool dr_faster(int64_t routes, int64_t experts, int64_t n, int64_t k, bool silu, bool prepacked,
+               int block_m, int64_t cus) {
   const double avg = (double)routes / (double)experts;
-  const int64_t nbn = (n + (silu ? 127 : 255)) / (silu ? 128 : 256);
-  const int64_t cus = device_cus();
+  const int64_t busy = std::min(routes, experts);
+  const int64_t wide = (n + (silu ? 127 : 255)) / (silu ? 128 : 256);  // column tiles
+  const int64_t narrow = (n + (silu ? 63 : 127)) / (silu ? 64 : 128);
   // a grid of less than two 256-column tiles per CU when every expert has
   // one block
-  const bool small = std::min(routes, experts) * nbn < 2 * cus;
+  const bool small = busy * wide < 2 * cus;
+  // 128-row blocks leave half of the CUs idle (long K only)
+  const bool idle = k >= 2048 && 2 * dr_blocks(routes, experts, 128) * wide <= cus;
   if (!prepacked) {
-    // Checkpoint layout.  Up to 1.5 routes per expert the 16-row decode
-    // kernels (soft op, E=128 K=2048 N=1536, 24 tokens 41.9 vs 44.4; 32
-    // tokens 46.8 -> 45.0, 48 52.1 -> 46.3).  Above 80 the 128-row
-    // persistent tiles on full grids of long K (MoE layer, E=128, 1024 /
-    // 1536 tokens 156.5 -> 152.0 / 173.3 vs 178.8; K=768 N=2048 at 96 / 128
-    // routes per expert 75.3 / 86.6 -> 69.3 / 84.7), above 128 on small ones
-    // too (E=32 top-4 layer, 128 / 256 routes per expert 94.1 -> 72.7 /
-    // 115.6 vs 124.3) unless even their 128-row blocks leave CUs idle (E=8
-    // top-2, I=1408, 256 routes per expert 93.7 -> 69.7).
-    // The layer keeps them up to 2.5 while its experts fill less than half
-    // the CUs (E=64 top-6 at 2 routes per expert, H x I 2048x512 / 1024x1408 /
-    // 4096x512 / 2048x1024 35.2 / 44.3 / 60.9 / 57.5 vs 36.9 / 45.8 / 62.7 /
-    // 55.0; E=128 H=2048 I=768 79.6 -> 75.0; E=64 at 3, H=4096 I=1024 108.1 ->
-    // 96.5).
-    if (avg <= (silu && 2 * std::min(routes, experts) < cus ? 2.5 : 1.5)) return false;
-    if (avg <= ((small || k < 2048) ? 128.0 : 80.0)) return true;
-    return dr_blocks(routes, experts, 128) * nbn < cus;
+    if (avg <= 1.5) return false;
+    if (block_m == 16) {
+      // Against the decode kernels, whose workgroups split K: not on grids of
+      // less than two 128-column tiles per CU (soft op, 32x2048x1536 at 3 / 4
+      // 21.8 / 22.9 vs 23.9 / 24.0, skewed 16.4 / 19.2 vs 21.1 / 22.2; layer,
+      // 32x2048x768 at 3 / 6 34.0 / 35.9 vs 36.7 / 37.4), and from 2.5 routes
+      // per expert unless the experts cover half of the CUs (soft op,
+      // 64x4096x1024 at 2 / 3 37.5 vs 38.9 / 43.0 -> 40.2; layer,
+      // 64x1024x1408 at 2 44.3 vs 45.8; 64x1024x512 26.3 -> 24.5 and
+      // 64x2048x1024 57.5 -> 55.0 at 2 are given up; 128x2048x768 at 2 / 3
+      // 79.8 / 86.3 -> 76.4 / 80.5)
+      return busy * narrow >= 2 * cus && (avg > 2.5 || 2 * busy >= cus);
+    }
+    if (block_m % 128 == 0) {
+      // Against 128-row tiles: on small grids up to 128 routes per expert
+      // (32x2048x1536 at 96 / 128 41.2 / 54.8 -> 32.7 / 47.9) and while even
+      // those tiles leave CUs idle (16x2048x1536 at 192 40.0 -> 30.8); on
+      // full grids less the shorter K is (64x768x2048 at 48 / 64 28.6 -> 27.7
+      // / 29.1 vs 30.9; 128x2048x1536 at 48 / 80 87.8 -> 82.3 / 93.4 vs 95.3;
+      // 128x4096x1024 at 80 / 96 143.3 -> 132.3 / 146.6 vs 145.1)
+      if (small) return avg <= 128.0 || dr_blocks(routes, experts, 128) * wide < cus;
+      return avg <= (k >= 4096 ? 80.0 : (k >= 2048 ? 64.0 : 48.0));
+    }
+    if (block_m % 64 != 0 && k < 2048) {
+      // 32-row tiles, short K: 64x768x2048 at 20 / 32 / 48 21.4 / 24.5 ->
+      // 17.7 / 21.6 / 28.6 vs 29.4; 8x768x2048 at 64 / 128 9.8 -> 9.1 / 11.4
+      // vs 11.6
+      return avg <= (busy * wide < cus ? 64.0 : 32.0);
+    }
+    if (block_m % 64 == 0 && !dr_wide(routes, experts, n, silu, 64, cus) && avg > 96.0) {
+      // 64-row tiles of the same grid, many rows: only where CUs idle
+      // (8x4096x1024 at 128 41.5 -> 31.2; 8x768x2048 at 96 / 128 11.1 -> 10.8
+      // / 12.1 vs 13.4; 16x2048x1536 at 192 30.3 vs 31.3)
+      return idle;
+    }
+    // full grids of long K up to 80 (128x2048x1536 at 64 / 80 / 96 1.10 / 1.15
+    // / 1.14 times as fast on a caller's 64-row blocks, 1.00 / 1.06 / 1.05 on
+    // 32-row ones; 64x2048x1536, 32-row, at 96 68.2 vs 68.6)
+    return avg <= ((small || k < 2048) ? 128.0 : 80.0) || idle;
   }
-  // Prepacked (MoE layer).  Against the 16-row decode kernels: 16 / 24
-  // tokens of E=128 63.5 / 74.5 -> 58.1 / 69.3.  On small grids up to 96
-  // routes per expert (E=8 top-2 I=1408 at 16 / 48 / 96: 37.3 / 52.5 / 53.9
-  // -> 29.6 / 41.5 / 45.0; 128: 55.4 vs 56.1; E=32 top-4 I=768 at 8 / 48 /
-  // 96: 34.3 / 52.3 / 61.6 -> 30.8 / 46.0 / 61.8).  On full ones 32-row
-  // prefill tiles up to 20 routes per expert, while their grid is one round
-  // (128 / 256 tokens of E=128 77.0 / 79.4 vs 75.4 / 81.4), this up to 32
-  // (384 / 512 tokens 92.4 / 94.1 -> 86.2 / 93.3), then 64-row prefill tiles
-  // (768 / 1024 tokens 115.0 / 130.6 vs 117.3 / 148.0).
+  // Prepacked (MoE layer).  Against the 16-row decode kernels at <= 1.5 routes
+  // per expert: 16 / 24 tokens of 128x2048x768 63.5 / 74.5 -> 58.1 / 69.3.
   if (avg <= 1.5) return true;
-  if (small) return avg > 2.0 && avg <= 96.0;
+  // Grids of less than 1.5 64-column tiles per CU: 16x2048x768 at 6 / 16 / 32
+  // / 64 / 96 33.9 / 34.4 / 35.4 / 52.4 / 53.2 -> 28.4 / 29.2 / 32.0 / 46.1 /
+  // 46.8.
+  if (2 * busy * narrow < 3 * cus) return avg > 2.0 && avg <= 96.0;
+  // Others: the 32-row tiles, whose grid is one round, up to ~28 routes per
+  // expert on small ones (32x2048x768 at 8 / 16 / 28 35.9 / 37.1 / 39.8 vs
+  // 35.0 / 36.5 / 40.5, skewed 36.4 / 38.1 / 42.2 vs 44.8 / 45.4 / 47.6; at 32
+  // 44.5 -> 41.4, skewed 43.0 -> 47.1), then this up to 64 where its tiles are
+  // at most one per CU (32x2048x768 at 48 / 64 / 96 54.7 / 58.4 -> 49.3 / 58.1
+  // / 61.7 vs 62.4; 64x2048x768, with 1.5, 79.2 vs 87.6 at 64); K >= 4096 at 4
+  // / 8 59.8 / 60.5 -> 56.2 / 57.6 (32x4096x1024).  On full ones this from 20
+  // to 32 (128x2048x768 at 20 / 24 / 32 / 40 82.4 vs 86.3 / 95.4 / 94.9 ->
+  // 87.2 / 94.1 / 102.7 vs 107.3; 128x4096x1024 at 24 / 32 224.6 / 240.9 ->
+  // 198.6 / 210.9).  Skewed routing turns 24 to 32 round on short K
+  // (128x2048x768 84.1 / 111.7 -> 94.3 / 116.9; 128x4096x1024 0.96 / 1.00 of
+  // the rate): the host does not know the counts.
+  if (small) {
+    if (busy * wide <= cus && ((avg > 28.0 && avg <= 64.0) || (k >= 4096 && avg > 2.0 && avg <= 8.0)))
+      return true;
+    return avg > 28.0 && avg <= 32.0;
+  }
   return avg > 20.0 && avg <= 32.0;
 }
 
-// 256-column tiles once there are two for every CU (E=64 K=4096 N=1024, 16 /
-// 64 / 96 routes per expert: 42.5 / 72.8 / 75.7 us against 40.4 / 67.1 / 93.2
-// on 128-column ones; E=128 K=2048 N=1536 52.1 against 57.0 at 16).
 int launch_w4a16_dr(const GemmArgs& g, int dtype, int epi, hipStream_t st) {
   const int bm = g.block_m % 64 == 0 ? 64 : 32;
-  const int out = epi == EPI_SILU_MUL ? 128 : 256;
-  const bool wide = dr_blocks(g.num_valid, g.num_experts, bm) * ((g.n + out - 1) / out) >=
-                        2 * (int64_t)device_cus() &&
+  const bool wide = dr_wide(g.num_valid, g.num_experts, g.n, epi == EPI_SILU_MUL, bm,
+                            device_cus()) &&
                     dr_lds(bm, 256, g.bs_n) <= kDrLds;
   if (dtype == MXFP4_DT_BF16) {
     switch (epi) {
@@ -524,3 +584,16 @@ int launch_w4a16_dr(const GemmArgs& g, int dtype, int epi, hipStream_t st) {
 }
 
 }  // namespace mx
+
+// For the tests (not in the public header): columns of the tile a routed GEMM
+// on blocks of block_m rows gets on a chip of `cus` CUs, 0 where it stays on
+// the other kernels.  rows: of this kernel's tiles, 32 or 64.
+extern "C" int mxfp4_test_dr_columns(int64_t routes, int64_t experts, int64_t n, int64_t k,
+                                     int silu, int prepacked, int block_m, int rows, int64_t cus) {
+  using namespace mx;
+  if (!dr_faster(routes, experts, n, k, silu, prepacked, block_m, cus) ||
+      dr_lds(64, 128, k / 32) > kDrLds)
+    return 0;
+  return dr_wide(routes, experts, n, silu, rows, cus) && dr_lds(rows, 256, k / 32) <= kDrLds ? 256
+                                                                                            : 128;
+}

@@ -961,7 +961,7 @@ extern "C" int mxfp4_moe_gemm_pre(const void* a, int a_dtype, int64_t a_rows,
   set_prepacked(g, pre_b, pre_s, n, k);
   const SoftPath path = soft_path(a_dtype, c_dtype, pre_b != nullptr);
   g.dr = (path == SOFT_W4A16 || path == SOFT_F32_W4A16) && block_m % 32 == 0 && dr_supported(g) &&
-         dr_faster(num_valid, num_experts, n, k, false, false);
+         dr_faster(num_valid, num_experts, n, k, false, false, block_m, device_cus());
   return dispatch_gemm(g, a_dtype, c_dtype, EPI_STORE, static_cast<hipStream_t>(stream));
 }
 
@@ -1040,7 +1040,8 @@ extern "C" int mxfp4_fused_moe_pre(const void* a, int a_dtype, int64_t a_rows,
                                    a_scale, b_scale, topk_weights, mul_routed_weight, nullptr,
                                    nullptr, nullptr, routes, 64, routes, top_k);
     const SoftPlan q = plan_soft(routes, num_experts, path, k, true);
-    dr = dr_supported(g) && dr_faster(routes, num_experts, n, k, false, false) &&
+    dr = dr_supported(g) &&
+         dr_faster(routes, num_experts, n, k, false, false, p.block_m, device_cus()) &&
          workspace_bytes >= q.total;
     if (dr) p = q;
   }
@@ -1325,7 +1326,8 @@ extern "C" int mxfp4_moe_layer_pre(const void* x, int x_dtype, int64_t m, int64_
   g2.pre_s = pre2_s;
   g2.pre_b_e = prepacked_nibble_bytes(hidden, inter);
   g2.pre_s_e = prepacked_scale_bytes(hidden, inter);
-  if (!direct && dr_faster(p.routes, num_experts, inter, hidden, true, pre13_b != nullptr)) {
+  if (!direct && dr_faster(p.routes, num_experts, inter, hidden, true, pre13_b != nullptr,
+                           p.block_m, device_cus())) {
     // both GEMMs on 64-row blocks of w4a16_dr, where its routing fits the
     // workspace
     const LayerPlan q = plan_layer(m, top_k, num_experts, hidden, inter, 2, pre13_b != nullptr, true);

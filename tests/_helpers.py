@@ -4,9 +4,12 @@ BASELINE distributions: codes uniform over 0..15, E8M0 scales uniform over
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import torch
 
+from mxfp4_amd import _lib
 from oracle import mxfp4_oracle as O
 
 
@@ -21,10 +24,30 @@ def rand_act(seed: int, shape, dtype=torch.bfloat16) -> torch.Tensor:
     return torch.randn(shape, generator=g).to(dtype)
 
 
+def dr_columns(routes, experts, n, k, *, block_m, rows=64, silu=False, prepacked=False,
+               cus=256) -> int:
+    """Tile columns (128 or 256) of the register-weight routed GEMM where the
+    dispatch rule takes it for these sizes, 0 where it does not; block_m: the
+    caller's blocks, or the ones the call would plan without that kernel."""
+    f = _lib.load().mxfp4_test_dr_columns
+    f.argtypes = [ctypes.c_int64] * 4 + [ctypes.c_int] * 4 + [ctypes.c_int64]
+    return f(routes, experts, n, k, silu, prepacked, block_m, rows, cus)
+
+
 def cuda(a) -> torch.Tensor:
     if isinstance(a, np.ndarray):
         a = torch.from_numpy(np.ascontiguousarray(a))
     return a.to("cuda")
+
+
+def shifted(t: torch.Tensor) -> torch.Tensor:
+    """The same bytes at an address 4 past a 16-byte boundary: as scale bytes,
+    the register-weight routed GEMM does not take them (the prefill tiles do)."""
+    buf = torch.empty(t.numel() + 16, dtype=t.dtype, device=t.device)
+    s = buf[4:4 + t.numel()].view(t.shape)
+    s.copy_(t)
+    assert s.data_ptr() % 16 == 4 and s.is_contiguous()
+    return s
 
 
 def _format_floor(o: np.ndarray, fmt: str) -> float:
