@@ -171,16 +171,18 @@ def test_registered_dense_copy_serves_the_reference_signature():
         P.unregister_prepacked(w)
 
 
-# AITER's entry with BLOCK_SIZE_M 32, E=128, top-8.  1024 tokens: more than
-# ten 32 x 128 tiles per CU, so the checkpoint layout runs 32 x 256 tiles
-# with 2-stage weight-line groups; 256 tokens (16 routes per expert): 32 x
-# 128 tiles with 4-stage groups.  The registered prepacked copy runs its own
-# 32-row tiles; bitwise the same C, and sampled rows on the FP64 oracle
+# AITER's entry with BLOCK_SIZE_M 32, E=128, top-8, scale bytes off a 16-byte
+# boundary (the prefill tiles; the aligned ones run the register-weight
+# kernel).  1024 tokens: more than ten 32 x 128 tiles per CU, so the
+# checkpoint layout runs 32 x 256 tiles with 2-stage weight-line groups; 256
+# tokens (16 routes per expert): 32 x 128 tiles with 4-stage groups.  The
+# registered prepacked copy runs its own 32-row tiles; bitwise the same C from
+# all three, and sampled rows on the FP64 oracle
 @pytest.mark.parametrize("m", [1024, 256])
 def test_routed_32x256_line_groups_bitwise(m):
     from mxfp4_amd import prepack as P
     from oracle import mxfp4_oracle as O
-    from _helpers import assert_parity
+    from _helpers import assert_parity, dr_columns, shifted
     print(f"routed 32-row line groups m={m}", flush=True)
     rng = np.random.default_rng(m)
     e, top_k, k, n = 128, 8, 2048, 1536
@@ -193,19 +195,21 @@ def test_routed_32x256_line_groups_bitwise(m):
     srt, eid, npp = mx.make_routing_device(ids, e, 32)
     one, ones_e = torch.ones(1, device="cuda"), torch.ones(e, device="cuda")
 
-    def run():
+    def run(scales):
         C = torch.full((m, top_k, n), 3.0, dtype=torch.bfloat16, device="cuda")
-        mx.fused_moe_mxfp4(a, B, C, one, ones_e, None, Bs, tw, ids, srt, eid, npp, True, top_k,
+        mx.fused_moe_mxfp4(a, B, C, one, ones_e, None, scales, tw, ids, srt, eid, npp, True, top_k,
                            False, False, {"BLOCK_SIZE_M": 32}, torch.bfloat16)
         return C
-    plain = run()
+    assert dr_columns(m * top_k, e, n, k, block_m=32, rows=32)
+    plain = run(shifted(Bs))
+    direct = run(Bs)
     P.register_prepacked(B, Bs)
     try:
-        fast = run()
+        fast = run(Bs)
     finally:
         P.unregister_prepacked(B)
     torch.cuda.synchronize()
-    assert torch.equal(plain, fast)
+    assert torch.equal(plain, fast) and torch.equal(plain, direct)
     rows = np.arange(0, m, 53 if m > 512 else 13)
     oracle = O.fused_moe_fp64(a.float().cpu().numpy()[rows], wp, ws, 1.0, np.ones(e),
                               tw.cpu().numpy()[rows], ids.cpu().numpy()[rows], True)
@@ -216,12 +220,14 @@ def test_routed_32x256_line_groups_bitwise(m):
 # (K / 64 = 6 or 10 stages: the last group's load covers two stages that do
 # not exist, reading the next row's bytes or zeros past the buffer, which no
 # stage uses) and a ragged last column tile (N = 200): 12.5 routes per
-# expert on 32-row blocks take the 32 x 128 tiles with 4-stage groups
+# expert on 32-row blocks take the 32 x 128 tiles with 4-stage groups where
+# the scale bytes are off a 16-byte boundary, and the register-weight kernel
+# where they are on one
 @pytest.mark.parametrize("k", [384, 640])
 def test_routed_line_groups_partial_last_group(k):
     from mxfp4_amd import prepack as P
     from oracle import mxfp4_oracle as O
-    from _helpers import assert_parity
+    from _helpers import assert_parity, dr_columns, shifted
     print(f"routed 4-stage line groups k={k}", flush=True)
     rng = np.random.default_rng(k)
     m, e, top_k, n = 100, 16, 2, 200
@@ -234,19 +240,21 @@ def test_routed_line_groups_partial_last_group(k):
     srt, eid, npp = mx.make_routing_device(ids, e, 32)
     one, ones_e = torch.ones(1, device="cuda"), torch.ones(e, device="cuda")
 
-    def run():
+    def run(scales):
         C = torch.full((m, top_k, n), 3.0, dtype=torch.bfloat16, device="cuda")
-        mx.fused_moe_mxfp4(a, B, C, one, ones_e, None, Bs, tw, ids, srt, eid, npp, True, top_k,
+        mx.fused_moe_mxfp4(a, B, C, one, ones_e, None, scales, tw, ids, srt, eid, npp, True, top_k,
                            False, False, {"BLOCK_SIZE_M": 32}, torch.bfloat16)
         return C
-    plain = run()
+    assert dr_columns(m * top_k, e, n, k, block_m=32, rows=32)
+    plain = run(shifted(Bs))
+    direct = run(Bs)
     P.register_prepacked(B, Bs)
     try:
-        fast = run()
+        fast = run(Bs)
     finally:
         P.unregister_prepacked(B)
     torch.cuda.synchronize()
-    assert torch.equal(plain, fast)
+    assert torch.equal(plain, fast) and torch.equal(plain, direct)
     oracle = O.fused_moe_fp64(a.float().cpu().numpy(), wp, ws, 1.0, np.ones(e),
                               tw.cpu().numpy(), ids.cpu().numpy(), True)
     assert_parity(plain.float().cpu().numpy(), oracle, what=f"4-stage groups k={k}")
