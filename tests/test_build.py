@@ -13,6 +13,14 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
+def _remarks(*sizes):
+    """As the compiler reports them, one kernel per size of scratch."""
+    return "".join(f"a.hip:3:1: remark: Function Name: kernel{i} [-Rpass-analysis]\n"
+                   f"a.hip:3:1: remark:     ScratchSize [bytes/lane]: {v} [-Rpass-analysis]\n"
+                   f"a.hip:3:1: remark:     SGPRs Spill: 0 [-Rpass-analysis]\n"
+                   for i, v in enumerate(sizes))
+
+
 @pytest.fixture
 def build(tmp_path, monkeypatch):
     """build.py with every output under tmp_path and commands that only write
@@ -26,12 +34,13 @@ def build(tmp_path, monkeypatch):
     monkeypatch.setattr(mod, "OBJ_DIR", str(tmp_path))
     monkeypatch.setattr(mod, "GEN_DIR", str(tmp_path))
     mod.fail = ()
+    mod.remarks = _remarks(0, 0)
 
     def run(cmd, **kw):
         if any(f in c for f in mod.fail for c in cmd):
             return subprocess.CompletedProcess(cmd, 1, "", "made to fail")
         open(cmd[cmd.index("-o") + 1], "w").close()
-        return subprocess.CompletedProcess(cmd, 0, "", "")
+        return subprocess.CompletedProcess(cmd, 0, "", mod.remarks)
 
     monkeypatch.setattr(mod.subprocess, "run", run)
     return mod
@@ -48,3 +57,13 @@ def test_failing_host_compiler_is_reported_after_the_library(build):
     with pytest.raises(RuntimeError, match="mxfp4_host.cpp"):
         build.build()
     assert os.path.exists(build.LIB) and os.path.exists(build.PROBE_LIB)
+
+
+@pytest.mark.parametrize("remarks,what", [(_remarks(0, 24, 0), r"kernel1 \(24 bytes/lane\)"),
+                                          ("", "no resource usage")])
+def test_scratch_in_a_kernel_that_counts_loads_fails_the_build(build, remarks, what):
+    assert all(os.path.exists(os.path.join(build.CSRC, f)) for f in build.NO_SCRATCH)
+    build.remarks = remarks
+    with pytest.raises(RuntimeError, match=what):
+        build.build()
+    assert not os.path.exists(build.LIB)
