@@ -207,6 +207,8 @@ __global__ __launch_bounds__(256) void align_place(const TI* __restrict__ ids, i
 // x % gridDim.x == c, and workgroup 0 the padded route count; small routings
 // launch kOneLeast workgroups for that (with one, its 8 waves walk 16
 // experts' padding each: 256 routes 7.9 us, with 16 to 64 workgroups 4.3).
+// One chunk (ONE) has no routes outside it: every workgroup takes its counts,
+// the first places it, and a workgroup for every 8 experts is enough.
 // Latency bound: a round of id loads per 8192 routes, three barriers, one
 // round of stores.  Graph replays of the call, 129 experts, 64-row blocks,
 // 1024 / 4096 / 8192 / 16384 routes: uniform ids 5.6 / 6.0 / 6.4 / 8.2 us,
@@ -215,14 +217,15 @@ __global__ __launch_bounds__(256) void align_place(const TI* __restrict__ ids, i
 // against 7.2 / 7.8 and 6.8 / 9.2 us in one workgroup up to 4096 routes (all
 // phases on one CU) and 9.4 / 9.3 and 9.5 / 9.4 us for the count and scan +
 // place launches, which win above (32768 uniform routes, where every
-// workgroup counts every id, 10.4 us against 7.8).  8 experts, 256 routes:
-// 5.2 us against 5.0 in one workgroup of 256 threads.
+// workgroup counts every id, 10.4 us against 7.8).  64 / 512 routes of 9
+// experts 3.6 / 3.7 us, of 129 3.9 / 4.0 (4.4 / 4.4, 4.7 / 4.8 with the counting
+// loop; one workgroup of 256 threads 3.6 / 4.2, 4.6 / 6.4), 513 of 9 4.5 (4.2).
 constexpr int kOneChunk = 512;
 constexpr int64_t kOneLeast = 16;
 constexpr int64_t kOneLaunch = 16384;
 constexpr int kOneCopies = 4;
 
-template <typename TI>
+template <typename TI, bool ONE>
 __global__ __launch_bounds__(kOneChunk) void align_one(const TI* __restrict__ ids, int64_t n,
                                                        int num_experts, int drop_to, int id_bits,
                                                        int block_m,
@@ -234,7 +237,7 @@ __global__ __launch_bounds__(kOneChunk) void align_one(const TI* __restrict__ id
   constexpr int B = 16;                  // id loads per thread per round trip
   __shared__ int wpos[W * kMaxExperts];  // [wave][expert]: counts, then next positions
   // [copy][expert]: routes of earlier (low half) and of later chunks (high)
-  __shared__ uint32_t cnt[kOneCopies * (kMaxExperts + 1)];
+  __shared__ uint32_t cnt[ONE ? 1 : kOneCopies * (kMaxExperts + 1)];
   __shared__ int s_start[kMaxExperts], s_fill[kMaxExperts];  // first slot, first sentinel slot
   __shared__ int part[W];
   const int tid = threadIdx.x;
@@ -244,15 +247,17 @@ __global__ __launch_bounds__(kOneChunk) void align_one(const TI* __restrict__ id
   const int ne = num_experts;
   const int stride = ne | 1;
   uint32_t* const my_cnt = cnt + (lane % kOneCopies) * stride;
-  const int64_t mine = (int64_t)c * NT + tid;
+  const int64_t mine = (int64_t)(ONE ? 0 : c) * NT + tid;
   const int eid = mine < n ? route_expert(ids[mine], ne, drop_to) : -1;
   TI v[B];
+  if constexpr (!ONE) {
 #pragma unroll
-  for (int b = 0; b < B; ++b) v[b] = (int64_t)b * NT + tid < n ? ids[b * NT + tid] : (TI)0;
+    for (int b = 0; b < B; ++b) v[b] = (int64_t)b * NT + tid < n ? ids[b * NT + tid] : (TI)0;
+    for (int i = tid; i < kOneCopies * stride; i += NT) cnt[i] = 0;
+  }
   for (int i = tid; i < W * ne; i += NT) wpos[i] = 0;
-  for (int i = tid; i < kOneCopies * stride; i += NT) cnt[i] = 0;
   __syncthreads();
-  for (int64_t i0 = 0; i0 < n; i0 += B * NT) {
+  for (int64_t i0 = 0; !ONE && i0 < n; i0 += B * NT) {
     if (i0 > 0) {
 #pragma unroll
       for (int b = 0; b < B; ++b) {
@@ -288,7 +293,7 @@ __global__ __launch_bounds__(kOneChunk) void align_one(const TI* __restrict__ id
     if (x < ne) {
       uint32_t others = 0;
 #pragma unroll
-      for (int q = 0; q < kOneCopies; ++q) others += cnt[q * stride + x];
+      for (int q = 0; q < (ONE ? 0 : kOneCopies); ++q) others += cnt[q * stride + x];
       pre[jj] = (int)(others & 0xFFFF);
       tot[jj] = pre[jj] + (int)(others >> 16);
 #pragma unroll
@@ -325,7 +330,7 @@ __global__ __launch_bounds__(kOneChunk) void align_one(const TI* __restrict__ id
   }
   if (c == 0 && tid == NT - 1) num_post_padded[0] = sum;
   __syncthreads();
-  if (eid >= 0) sorted_ids[wpos[wave * ne + eid] + rank] = (int32_t)mine;
+  if (eid >= 0 && (!ONE || c == 0)) sorted_ids[wpos[wave * ne + eid] + rank] = (int32_t)mine;
   for (int x = c + wave * nwg; x < ne; x += W * nwg) {
     const int st = s_start[x], fill = s_fill[x];
     const int blocks = (fill - st + block_m - 1) / block_m;
@@ -555,8 +560,15 @@ int launch_align(const TI* ids, int64_t n, int num_experts, int drop_to, int blo
   while ((1 << id_bits) < num_experts) ++id_bits;
   if (n <= kOneLaunch) {
     const int64_t chunks = (n + kOneChunk - 1) / kOneChunk;
-    align_one<TI><<<(unsigned)(chunks > kOneLeast ? chunks : kOneLeast), kOneChunk, 0, st>>>(
-        ids, n, num_experts, drop_to, id_bits, block_m, sorted_ids, expert_ids, npp);
+    if (chunks <= 1) {
+      const int64_t nwg = (num_experts + kOneChunk / 64 - 1) / (kOneChunk / 64);
+      align_one<TI, true><<<(unsigned)(nwg < kOneLeast ? nwg : kOneLeast), kOneChunk, 0, st>>>(
+          ids, n, num_experts, drop_to, id_bits, block_m, sorted_ids, expert_ids, npp);
+    } else {
+      align_one<TI, false>
+          <<<(unsigned)(chunks > kOneLeast ? chunks : kOneLeast), kOneChunk, 0, st>>>(
+              ids, n, num_experts, drop_to, id_bits, block_m, sorted_ids, expert_ids, npp);
+    }
     return launch_status("align launch");
   }
   if (nchunks > 0) {

@@ -17,8 +17,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("routes,num_experts,block_m",
-                         [(1, 1, 16), (63, 1024, 16), (511, 128, 64), (512, 128, 64),
-                          (513, 129, 32), (8191, 3, 48), (8193, 1024, 16), (16383, 64, 128),
+                         [(1, 1, 16), (63, 1024, 16), (64, 9, 64), (300, 17, 32),
+                          (511, 128, 64), (512, 128, 64), (513, 129, 32), (8191, 3, 48), (8193, 1024, 16), (16383, 64, 128),
                           (16384, 257, 64), (16385, 128, 64)])
 @pytest.mark.parametrize("skew", [False, True])
 def test_one_launch_routing_matches_host_loop(routes, num_experts, block_m, skew):
