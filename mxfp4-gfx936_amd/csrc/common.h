@@ -93,11 +93,11 @@ __device__ __forceinline__ void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// Calls f(std::integral_constant<int, I>{}) for I = B .. E-1 (compile-time
-// indices for register arrays and template arguments inside loops).
 // Every LDS read this wave has issued has returned.
 __device__ __forceinline__ void wait_lgkm0() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
+// Calls f(std::integral_constant<int, I>{}) for I = B .. E-1 (compile-time
+// indices for register arrays and template arguments inside loops).
 template <int B, int E, typename F>
 __device__ __forceinline__ void static_for(F&& f) {
   if constexpr (B < E) {

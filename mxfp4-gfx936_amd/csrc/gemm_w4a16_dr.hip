@@ -16,7 +16,10 @@
 //   v_permlane swaps per 16 bytes transpose the blocks over the lane groups
 //   into the order the prefill tiles multiply in.  The prepacked nibbles
 //   (PRE) are in that order already.  Either way the results are bitwise
-//   those of the prefill tiles.
+//   those of the prefill tiles.  They are not those of the 16-row decode
+//   kernels, which add K in another order: calls that this kernel takes from
+//   them (block_m 16 in dr_faster) differ by rounding, 2e-4 of the 2-norm in
+//   bf16, at the same error against 64 bits.
 // * The tile's E8M0 bytes (checkpoint layout in both cases) are one
 //   contiguous piece of the scale matrix (two with SiLU): copied to LDS once,
 //   by 1 KB wave-loads.
@@ -80,8 +83,6 @@ __device__ __forceinline__ void transpose_blocks(uint32_t (&d)[4]) {
     d[j + 1] = s[1];
   }
 }
-
-
 
 struct DrTile {
   int64_t pos0;
@@ -341,7 +342,7 @@ __global__ __launch_bounds__(256, FN == 2 ? 4 : 3) void w4a16_dr(GemmArgs g, int
   int bm, bn;
   if (!tile_of(g, BM, nbm, nbn, bm, bn, blockIdx.x, gridDim.x)) return;
   t.pos0 = (int64_t)bm * BM;
-  t.expert = g.sorted_ids ? block_expert(g, t.pos0) : 0;
+  t.expert = block_expert(g, t.pos0);
   t.ncol0 = bn * OUT_COLS;
   if (t.expert < 0) {  // aiter:156-172: expert not on this device -> zeros
     for (int idx = threadIdx.x; idx < BM * OUT_COLS; idx += 256) {

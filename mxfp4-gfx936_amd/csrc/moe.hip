@@ -1047,7 +1047,7 @@ extern "C" int mxfp4_fused_moe_pre(const void* a, int a_dtype, int64_t a_rows,
   // checkpoint-layout weights on 64-row blocks of w4a16_dr where it is faster
   // and its routing fits the workspace
   bool dr = false;
-  if ((path == SOFT_W4A16 || path == SOFT_F32_W4A16) && routes > 0 && routes > kDirectRoutes) {
+  if ((path == SOFT_W4A16 || path == SOFT_F32_W4A16) && routes > kDirectRoutes) {
     const GemmArgs g = routed_args(a, a_rows, a_row_stride, a_mx, b, b_mx, num_experts, n, k, c, n,
                                    a_scale, b_scale, topk_weights, mul_routed_weight, nullptr,
                                    nullptr, nullptr, routes, 64, routes, top_k);
