@@ -185,7 +185,8 @@ def unregister_prepacked(packed: torch.Tensor) -> None:
 
 
 def any_registered() -> bool:
-    """Whether any copy is registered (then the operators look theirs up)."""
+    """Whether any copy is registered: the operators whose signatures have no
+    place for a copy then look theirs up, on their general path."""
     return bool(_REGISTRY)
 
 
