@@ -499,7 +499,7 @@ bool dr_faster(int64_t routes, int64_t experts, int64_t n, int64_t k, bool silu,
   if (!prepacked) {
     if (avg <= 1.5) return false;
     if (block_m == 16) {
-      // Against the decode kernels, whose workgroups split K: not on grids of
+      // Against the decode kernels, whose waves split K: not on grids of
       // less than two 128-column tiles per CU (soft op, 32x2048x1536 at 3 / 4
       // 21.8 / 22.9 vs 23.9 / 24.0, skewed 16.4 / 19.2 vs 21.1 / 22.2; layer,
       // 32x2048x768 at 3 / 6 34.0 / 35.9 vs 36.7 / 37.4), and from 2.5 routes
